@@ -22,14 +22,20 @@ import torch
 from . import layout as L
 from .chain import Chain
 
+# One handle per device and stream: calls on a handle share its workspace, so
+# they have to be ordered.  The oldest goes when there are _MOST_CHAINS (its
+# memory is freed once the device has finished with it).
+_MOST_CHAINS = 64
 _chains = {}
 
 
 def _chain():
-    dev = torch.cuda.current_device()
-    if dev not in _chains:
-        _chains[dev] = Chain()
-    return _chains[dev]
+    key = torch.cuda.current_device(), torch.cuda.current_stream().cuda_stream
+    if key not in _chains:
+        if len(_chains) >= _MOST_CHAINS:
+            del _chains[next(iter(_chains))]
+        _chains[key] = Chain()
+    return _chains[key]
 
 
 def _scene(scene, state, temperature, pressure, qv):

@@ -278,8 +278,11 @@ __device__ __forceinline__ void cell_finish(const ChainArgs &a, long off, const 
       }
     }
   } else {
-    gi_out[F_H2SO4] = X.h3 * 1.0;
-    gi_out[F_SOAG] = X.s3 * 1.0;
+    // The diagnostics instantiation reads the two gases again: it keeps live
+    // values in accumulation registers across the clear subarea's code, and
+    // the compiler's copies there left out the overcast lanes.
+    gi_out[F_H2SO4] = (P::diag ? ld3w<P>(a, off, F_H2SO4, TO_VMR_H2SO4) : X.h3) * 1.0;
+    gi_out[F_SOAG] = (P::diag ? ld3w<P>(a, off, F_SOAG, TO_VMR_SOAG) : X.s3) * 1.0;
   }
 
   if (X.cat != 0) {

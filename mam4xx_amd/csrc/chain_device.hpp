@@ -375,6 +375,157 @@ __device__ __forceinline__ int soa_state_exp(const SoaState<double> &s) {
 }
 __device__ __forceinline__ int soa_state_exp(const SoaState<num::Dual> &) { return 0; }
 
+// ---- the FAST sub-step on bounded inputs
+// SoaRun is the loop of one cell whose inputs passed soa_run_ok: every mass is
+// 0 or in [2^-400, 2^8] to begin with, a skipped mode (uptake <= 1e-15) has
+// uk = a = 0, the loop runs at least one sub-step, and the two modes whose
+// oxygenated POM soa_in_state makes 0 have none.  The masses then stay
+// >= 0 and finite, so soa_run_tick leaves out the clips of a state at 0, the
+// skip selects and the leading 0 + x of the sums, and takes vmax for kmax (the
+// larger of three in any order): every value equals soa_tick<true>'s bit for
+// bit.
+//
+// low is the smallest high word minus one (unsigned, so that a zero counts as
+// large) among the states' masses: the record soa_fast_exact needs.  A state
+// in {0} u [2^-400, 2^11] is followed by one in {0} u [2^-968, 2^11] (the
+// bounds above), so a non-zero mass never has a zero high word before low has
+// seen one below 2^-400.
+template <int NM>
+struct SoaRun {
+  double g, a[NM], uk[NM], aopoa[NM], g0;
+  double tcur, avg, dtsum;
+  int niter;
+  unsigned low;
+  bool run;  // the loop goes on
+};
+constexpr unsigned kSoaLowMin = 0x26f00000u - 1u;  // high word of 2^-400, minus one
+
+__host__ __device__ constexpr bool soa_fresh(int mode) { return mode == NAIT || mode == NPCA; }
+__device__ __forceinline__ bool soa_mass_ok(double x) {
+  return x == 0.0 || (x >= 0x1p-400 && x <= 0x1p8);
+}
+// mode slot j of the run from the cell's inputs; returns whether its inputs
+// are in range
+// (fresh: the mode has no oxygenated POM)
+template <int NM>
+__device__ __forceinline__ bool soa_run_mode(SoaRun<NM> &s, int j, double a, double uptk,
+                                             double aopoa, bool fresh) {
+  const double uk = uptk * 0.81;  // gasaerexch.hpp:458-465
+  const bool skip = !(uk > 1.0e-15);
+  s.uk[j] = skip ? 0.0 : uk;
+  s.a[j] = skip ? 0.0 : a;
+  s.aopoa[j] = aopoa;
+  return s.uk[j] <= 0x1p60 && (fresh ? aopoa == 0.0 : ::fabs(aopoa) <= 0x1p10) &&
+         soa_mass_ok(s.a[j]);
+}
+template <int NM>
+__device__ __forceinline__ bool soa_run_cell(SoaRun<NM> &s, double g, double g0, double dtfull) {
+  s.g = g;
+  s.g0 = g0;
+  s.tcur = 0.0;
+  s.avg = 0.0;
+  s.dtsum = 0.0;
+  s.niter = 0;
+  s.run = true;
+  return dtfull >= 1.0 && dtfull <= 0x1p20 && soa_mass_ok(g) &&
+         (g0 == 0.0 || (g0 >= 0x1p-300 && g0 <= 0x1p10));
+}
+__device__ __forceinline__ void soa_run_init(SoaRun<4> &s, const SoaIn<double> &in,
+                                             double dtfull) {
+  bool ok = soa_run_cell(s, in.g, in.g0, dtfull);
+#pragma unroll
+  for (int n = 0; n < 4; ++n)
+    ok = soa_run_mode(s, n, in.a[n], in.uptk[n], in.aopoa[n], soa_fresh(n)) && ok;
+  s.low = ok ? 0xffffffffu : 0u;
+}
+template <int NM>
+__device__ __forceinline__ void soa_run_low(SoaRun<NM> &s) {
+  unsigned m = num::high_word(s.g) - 1u;
+#pragma unroll
+  for (int n = 0; n < NM; ++n) {
+    const unsigned h = num::high_word(s.a[n]) - 1u;
+    m = h < m ? h : m;
+  }
+  s.low = m < s.low ? m : s.low;
+}
+
+// Sums over a cell's four modes, in mode order: one lane holds them all, or
+// (NM = 1, GPU only) four neighbouring lanes hold one mode each and every lane
+// gets the sum.
+__device__ __forceinline__ double soa_sum(const double (&x)[4]) {
+  return ((x[0] + x[1]) + x[2]) + x[3];
+}
+__device__ __forceinline__ double soa_sum_from(double s, const double (&x)[4]) {
+  return (((s + x[0]) + x[1]) + x[2]) + x[3];
+}
+#if defined(__HIP__)
+template <int K>
+__device__ __forceinline__ double quad_lane(double x) {  // lane K of the four
+#if defined(__HIP_DEVICE_COMPILE__)
+  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(x), K * 0x55, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(x), K * 0x55, 0xf, 0xf, true);
+  return __hiloint2double(hi, lo);
+#else
+  return x;
+#endif
+}
+__device__ __forceinline__ double soa_sum(const double (&x)[1]) {
+  return ((quad_lane<0>(x[0]) + quad_lane<1>(x[0])) + quad_lane<2>(x[0])) + quad_lane<3>(x[0]);
+}
+__device__ __forceinline__ double soa_sum_from(double s, const double (&x)[1]) {
+  return (((s + quad_lane<0>(x[0])) + quad_lane<1>(x[0])) + quad_lane<2>(x[0])) +
+         quad_lane<3>(x[0]);
+}
+#endif
+
+// One sub-step of a SoaRun that runs: soa_tick<true>, with the loop's own test
+// after it instead of before.
+template <int NM>
+__device__ __forceinline__ void soa_run_tick(SoaRun<NM> &s, double dtfull) {
+  const double alpha_astem = 0.05, a_min1 = 1.0e-20, g_min1 = 1.0e-20;
+  const double g = s.g, gfloor = num::vmax(g, g_min1);
+  double sat[NM], del[NM], term[NM];
+#pragma unroll
+  for (int n = 0; n < NM; ++n) {
+    const double org = NM == 4 && soa_fresh(n) ? s.a[n] : s.aopoa[n] + s.a[n];
+    sat[n] = num::div_fast(s.g0, num::vmax(org, a_min1));
+    const double gstar = sat[n] * s.a[n];
+    del[n] = g - gstar;
+    const double phi = num::div_fast(del[n], num::vmax(gfloor, gstar));
+    term[n] = s.uk[n] * ::fabs(phi);
+  }
+  const double tot = soa_sum_from(g, s.a), tmpa = soa_sum(term);
+  const double dtmax = dtfull - s.tcur;
+  const bool last = dtmax * tmpa <= alpha_astem;
+  const double dtcur = last ? dtmax : num::div_fast(alpha_astem, tmpa);
+  s.tcur = last ? dtfull : s.tcur + dtcur;
+  double beta[NM], den[NM], r[NM], qa[NM], qb[NM];
+#pragma unroll
+  for (int n = 0; n < NM; ++n) {
+    beta[n] = dtcur * s.uk[n];
+    const double at = s.a[n] + beta[n] * del[n];
+    const double org = NM == 4 && soa_fresh(n) ? at : s.aopoa[n] + at;
+    const double sat1 = num::div_fast(s.g0, num::vmax(org, a_min1));
+    den[n] = 1.0 + beta[n] * (del[n] > 0.0 ? sat1 : sat[n]);
+    r[n] = num::rcp(den[n]);
+    qa[n] = num::div_r(s.a[n], den[n], r[n]);
+    qb[n] = num::div_r(beta[n], den[n], r[n]);
+  }
+  const double sa = soa_sum(qa), sb = soa_sum(qb);
+  const double gn = num::vmax(num::div_fast(tot - sa, 1.0 + sb), 0.0);
+#pragma unroll
+  for (int n = 0; n < NM; ++n)
+    s.a[n] = num::div_r(s.a[n] + beta[n] * gn, den[n], r[n]);
+  s.g = gn;
+  s.avg += dtcur * (g + 0.5 * (gn - g));
+  s.dtsum += dtcur;
+  soa_run_low(s);
+  // the reference counts the sub-step that its cap refuses
+  const bool more = s.tcur < dtfull - 1.0e-3, cap = s.niter >= 999;
+  s.niter += more && cap ? 2 : 1;
+  s.run = more && !cap;
+}
+
 // One cell's SOA loop from its inputs, equal bit for bit to the IEEE loop:
 // FAST sub-steps while soa_fast_exact holds, else the IEEE loop from the
 // start.

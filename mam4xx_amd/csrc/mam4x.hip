@@ -20,7 +20,7 @@
 //                         next cell as soon as its current one has converged
 //   4. chain_post_kernel  per cell: the rest of the chain, recombination,
 //                         calcsize, tendencies
-// chain_fused_kernel runs everything in one lane per cell (small domains).
+// chain_fused_kernel runs everything in one lane per cell (MAM4X_SCHED_FUSED).
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -94,38 +94,56 @@ constexpr unsigned char kCapped = 0x80;  // bucket bit: the SOA loop hit its cap
 constexpr unsigned char kIeee = 0x40;
 static_assert(kNBucket <= kIeee, "bucket indices stay below the flag bits");
 
-// Workspace: 14 planes of one double per cell.  The set-up kernel writes
-// them in cell order (coalesced); the queue kernel's chunks hold cells of a
-// few set-up blocks, so its gathers stay on few lines.
-//   plane 0 SOAG, 1..4 SOA per mode, 5 equilibrium SOAG g0,
-//   6..9 H2SO4 uptake rates, 10..13 oxygenated POM per mode.
-// The queue kernel overwrites planes 0..5 with its results: SOAG, SOA per
-// mode and the time-averaged SOAG.
-enum { W_G = 0, W_A = 1, W_G0 = 5, W_UPTK = 6, W_AOPOA = 10, W_NPLANE = 14 };
+// Workspace: a record of 14 doubles per cell, in cell order.
+//   0 SOAG, 1..4 SOA per mode, 5 equilibrium SOAG g0, 6..9 H2SO4 uptake
+//   rates, 10..13 oxygenated POM per mode.
+// The queue kernel overwrites 0..5 with its results: SOAG, SOA per mode and
+// the time-averaged SOAG.  It takes its cells in queue order, so a cell's
+// values lie together: two 64-byte lines a cell instead of one for each of
+// fourteen planes (21,600 x 72: 6.0x the loop's own bytes with planes).
+enum { W_G = 0, W_A = 1, W_G0 = 5, W_UPTK = 6, W_AOPOA = 10, W_REC = 14 };
 constexpr int W_GAVG = W_G0;
+struct __align__(16) Pair {
+  double x, y;
+};
+constexpr int kRecPairs = W_REC / 2;
 
-__device__ __forceinline__ void ws_store_in(double *ws, long n, long c,
-                                            const dev::SoaIn<double> &in) {
-  ws[W_G * n + c] = in.g;
-#pragma unroll
-  for (int m = 0; m < 4; ++m) {
-    ws[(W_A + m) * n + c] = in.a[m];
-    ws[(W_UPTK + m) * n + c] = in.uptk[m];
-    ws[(W_AOPOA + m) * n + c] = in.aopoa[m];
-  }
-  ws[W_G0 * n + c] = in.g0;
+__device__ __forceinline__ void ws_store_in(double *ws, long c, const dev::SoaIn<double> &in) {
+  Pair *p = reinterpret_cast<Pair *>(ws + c * W_REC);
+  p[0] = Pair{in.g, in.a[0]};
+  p[1] = Pair{in.a[1], in.a[2]};
+  p[2] = Pair{in.a[3], in.g0};
+  p[3] = Pair{in.uptk[0], in.uptk[1]};
+  p[4] = Pair{in.uptk[2], in.uptk[3]};
+  p[5] = Pair{in.aopoa[0], in.aopoa[1]};
+  p[6] = Pair{in.aopoa[2], in.aopoa[3]};
 }
 
-__device__ __forceinline__ void ws_load_in(const double *ws, long n, long c,
-                                           dev::SoaIn<double> &in) {
-  in.g = ws[W_G * n + c];
-#pragma unroll
-  for (int m = 0; m < 4; ++m) {
-    in.a[m] = ws[(W_A + m) * n + c];
-    in.uptk[m] = ws[(W_UPTK + m) * n + c];
-    in.aopoa[m] = ws[(W_AOPOA + m) * n + c];
-  }
-  in.g0 = ws[W_G0 * n + c];
+__device__ __forceinline__ void ws_load_in(const double *ws, long c, dev::SoaIn<double> &in) {
+  const Pair *p = reinterpret_cast<const Pair *>(ws + c * W_REC);
+  const Pair v[kRecPairs] = {p[0], p[1], p[2], p[3], p[4], p[5], p[6]};
+  in.g = v[0].x;
+  in.a[0] = v[0].y;
+  in.a[1] = v[1].x;
+  in.a[2] = v[1].y;
+  in.a[3] = v[2].x;
+  in.g0 = v[2].y;
+  in.uptk[0] = v[3].x;
+  in.uptk[1] = v[3].y;
+  in.uptk[2] = v[4].x;
+  in.uptk[3] = v[4].y;
+  in.aopoa[0] = v[5].x;
+  in.aopoa[1] = v[5].y;
+  in.aopoa[2] = v[6].x;
+  in.aopoa[3] = v[6].y;
+}
+
+__device__ __forceinline__ void ws_store_out(double *ws, long c, double g, const double a[4],
+                                             double gavg) {
+  Pair *p = reinterpret_cast<Pair *>(ws + c * W_REC);
+  p[0] = Pair{g, a[0]};
+  p[1] = Pair{a[1], a[2]};
+  p[2] = Pair{a[3], gavg};
 }
 
 struct QueueCtl {
@@ -155,13 +173,14 @@ static QueueShape queue_shape(const mam4x_config &c) {
 
 struct Work {
   QueueShape qs;
-  double *ws;              // W_NPLANE planes of ncell doubles
+  double *ws;              // ncell records of W_REC doubles
   unsigned char *bucket;   // per cell, kNoSoa when the cell has no SOA loop
   int *queue;              // cell indices, longest first
   QueueCtl *ctl;
   long ncell;              // cells of the launch (batches: padded to whole blocks)
   double dtfull;           // SOA loop length: the integer sub-step (:1319)
   unsigned long long *stats;  // SOA sub-step counter (NULL: off)
+  int quad;                // soa_queue_kernel starts in its QUAD form
 };
 
 // Where a block's cells come from.  A launch covers either one domain, or a
@@ -300,7 +319,7 @@ __global__ void __launch_bounds__(kBlock) chain_pre_kernel(Src src, Work w) {
       dev::clear_build<P>(a, off, X, S, G);
       dev::SoaIn<double> in;
       dev::clear_pre<P>(*a.K, X.T, X.p, X.dgw, S, G.g[0], in);
-      ws_store_in(w.ws, w.ncell, g, in);
+      ws_store_in(w.ws, g, in);
       dev::SoaState<double> st;
       dev::soa_init(st, in);
       const float pred = (float)dev::soa_predict(st, w.dtfull);
@@ -316,18 +335,28 @@ __global__ void __launch_bounds__(kBlock) chain_pre_kernel(Src src, Work w) {
 }
 
 // Phase 2: queue = cells grouped by bucket, highest bucket first.  Order
-// within a bucket is arbitrary; every cell's result is independent of it.
+// within a bucket is arbitrary; every cell's result is independent of it.  The
+// blocks' atomics on the 24 cursors serialise across the device, so a block
+// takes kScatter cells a lane (21,600 x 72: 74 us at one cell a lane, 19 us at
+// eight).
+constexpr int kScatter = 8;
+static unsigned scatter_grid(long ncell) {
+  return (unsigned)((ncell + kBlock * kScatter - 1) / (kBlock * kScatter));
+}
 __global__ void __launch_bounds__(kBlock) queue_scatter_kernel(Work w) {
   __shared__ unsigned cnt[kNBucket], base[kNBucket];
   if (threadIdx.x < kNBucket) cnt[threadIdx.x] = 0;
   __syncthreads();
-  const long c = (long)blockIdx.x * kBlock + threadIdx.x;
-  unsigned char b = kNoSoa;
-  unsigned r = 0;
-  if (c < w.ncell) {
-    b = w.bucket[c];
-    if (b != kNoSoa) r = atomicAdd(&cnt[b], 1u);
+  const long c0 = (long)blockIdx.x * kBlock * kScatter + threadIdx.x;
+  unsigned char b[kScatter];
+  unsigned r[kScatter];
+#pragma unroll
+  for (int j = 0; j < kScatter; ++j) {
+    const long c = c0 + (long)j * kBlock;
+    b[j] = c < w.ncell ? w.bucket[c] : kNoSoa;
   }
+#pragma unroll
+  for (int j = 0; j < kScatter; ++j) r[j] = b[j] != kNoSoa ? atomicAdd(&cnt[b[j]], 1u) : 0u;
   __syncthreads();
   if (threadIdx.x < kNBucket) {
     const int t = threadIdx.x;
@@ -336,99 +365,306 @@ __global__ void __launch_bounds__(kBlock) queue_scatter_kernel(Work w) {
     base[t] = cnt[t] ? start + atomicAdd(&w.ctl->fill[t], cnt[t]) : 0;
   }
   __syncthreads();
-  if (b != kNoSoa) w.queue[base[b] + r] = (int)c;
+#pragma unroll
+  for (int j = 0; j < kScatter; ++j)
+    if (b[j] != kNoSoa) w.queue[base[b[j]] + r[j]] = (int)(c0 + (long)j * kBlock);
 }
 
-// Phase 3: persistent SOA loop.  Each wave takes a chunk of queue entries at
-// a time (kChunk from the long part, kShortChunk from the short part); a lane
-// whose cell has converged takes the next entry of the wave's chunk before
-// the following sub-step.  A wave exits once the queue is exhausted and all
-// its lanes are idle; the queue is finite and every cell ends after at most
-// 1000 sub-steps, so every wave exits.
+// Phase 3: persistent SOA loop.  What bounds a cell is its chain of up to
+// 1000 dependent sub-steps (a lane alone: ~0.8 us each), and what bounds the
+// kernel is that no wave that carries such a chain waits for anything else.
+//
+//  * A lane whose cell has converged takes the wave's next cell.  The cells
+//    come from a segment of kSeg records in LDS; the following segment's
+//    records are in flight into registers and the one after that has its queue
+//    entries in flight, each a segment's work ahead, and so is the atomic that
+//    claims queue entries.  (A lane that gathered its next cell's inputs
+//    itself stalled the whole wave for it on most passes: with 27,648 cells,
+//    a wave each and nothing to wait for, 1.42 ms against 1.10.)
+//  * Refills wait for kRefill idle lanes.
+//  * QUAD form: four neighbouring lanes take a cell, one mode each, its sums
+//    through DPP in mode order (bit for bit the one-lane form).  A sub-step
+//    takes half as long, for twice the issue slots a cell.  Launches that do
+//    not fill the chip start in it (kQuadCells), and every wave
+//    turns to it when the queue is empty and at most 16 of its cells are left.
+//
+// A wave exits once the queue is exhausted and all its lanes are idle; the
+// queue is finite and every cell ends after at most 1000 sub-steps, so every
+// wave exits.
+constexpr int kSeg = 32;      // records staged at a time
+constexpr int kRefill = 4;    // idle lanes that trigger a refill
+constexpr int kWaves = kBlock / 64;
+constexpr int kQuadLanes = 16;  // cells of a wave in QUAD form
+
+// The wave's source of queue entries: a claimed range, the next claim's
+// atomic in flight.  The long part of the queue first (the first claim of
+// every wave static: claim = wave index), then the short part.
+struct Claims {
+  unsigned beg, end;  // what is left of the claimed range (wave-uniform)
+  unsigned pend;      // lane 0: the outstanding atomic's result
+  bool longs, over;
+  unsigned nq, nsplit, chunk, short_chunk, first;
+  QueueCtl *ctl;
+  int lane;
+  __device__ __forceinline__ void ask() {
+    if (lane == 0) pend = atomicAdd(longs ? &ctl->head : &ctl->shead, longs ? chunk : short_chunk);
+  }
+  __device__ __forceinline__ void init(unsigned wid, unsigned nwave) {
+    first = nwave * chunk;
+    longs = true;
+    over = false;
+    pend = 0;
+    beg = min(wid * chunk, nsplit);
+    end = min(beg + chunk, nsplit);
+    if (first >= nsplit) longs = false;  // the static claims cover the long part
+    if (!longs && nsplit == nq)
+      over = beg == end;
+    else
+      ask();
+  }
+  // the next range of at most kSeg entries (empty: none left)
+  __device__ __forceinline__ void next(unsigned &b, unsigned &e) {
+    while (beg == end && !over) {
+      if (!longs && nsplit == nq) {
+        over = true;
+        break;
+      }
+      const unsigned v = __builtin_amdgcn_readfirstlane(pend) + (longs ? first : nsplit);
+      const unsigned lim = longs ? nsplit : nq;
+      if (v < lim) {
+        beg = v;
+        end = min(v + (longs ? chunk : short_chunk), lim);
+        ask();
+      } else if (longs) {
+        longs = false;
+        if (nsplit < nq) ask();
+      } else {
+        over = true;
+      }
+    }
+    b = beg;
+    e = min(beg + kSeg, end);
+    beg = e;
+  }
+};
+
+// Records on their way from the queue to the wave's LDS segment.  Lane l moves
+// the pairs (l & 7) of records l / 8, l / 8 + 8, ...; the place after a
+// record's seven pairs carries the cell's index, and a record's places are
+// rotated by its number, so that lanes reading one value of neighbouring
+// records hit different banks.
+struct Staged {
+  int id[kSeg / 8];
+  Pair v[kSeg / 8];
+  __device__ __forceinline__ void ids(const int *queue, unsigned b, unsigned e, int lane) {
+#pragma unroll
+    for (int j = 0; j < kSeg / 8; ++j) id[j] = queue[min(b + 8 * j + (lane >> 3), e - 1)];
+  }
+  __device__ __forceinline__ void records(const double *ws, int lane) {
+#pragma unroll
+    for (int j = 0; j < kSeg / 8; ++j) {
+      const int c = ((lane & 7) - (lane >> 3)) & 7;  // 8 j + lane / 8 = lane / 8 mod 8
+      const Pair *p = reinterpret_cast<const Pair *>(ws + (long)id[j] * W_REC);
+      v[j] = p[c < kRecPairs ? c : 0];
+      if (c == kRecPairs) v[j].x = __hiloint2double(0, id[j]);
+    }
+  }
+  __device__ __forceinline__ void put(Pair *seg, int lane) const {
+#pragma unroll
+    for (int j = 0; j < kSeg / 8; ++j) seg[64 * j + lane] = v[j];
+  }
+};
+__device__ __forceinline__ Pair seg_pair(const Pair *seg, int r, int c) {
+  return seg[8 * r + ((c + r) & 7)];
+}
+__device__ __forceinline__ double seg_value(const Pair *seg, int r, int f) {
+  const double *q = reinterpret_cast<const double *>(seg + 8 * r + (((f >> 1) + r) & 7));
+  return q[f & 1];
+}
+__device__ __forceinline__ int seg_cell(const Pair *seg, int r) {
+  return __double2loint(seg_value(seg, r, W_REC));
+}
+
+// a finished cell's flags in its bucket byte (buckets are < kIeee; the set-up
+// kernel rewrites it every step); whether its results stand.  Flagged kIeee it
+// keeps its inputs, for soa_ieee_kernel.
+__device__ __forceinline__ bool soa_done(const Work &w, int cell, int niter, unsigned low) {
+  if (low < dev::kSoaLowMin) {
+    w.bucket[cell] = (unsigned char)(w.bucket[cell] | kIeee);
+    return false;
+  }
+  if (niter > 1000) w.bucket[cell] = (unsigned char)(w.bucket[cell] | kCapped);
+  return true;
+}
+__device__ __forceinline__ double soa_mean(double avg, double dtsum) {
+  return dev::kmax(0.0, avg / dtsum);
+}
+
 __global__ void __launch_bounds__(kBlock) soa_queue_kernel(Work w, unsigned long long *stats) {
+  __shared__ Pair lds[kWaves][kSeg * 8];
+  const int lane = threadIdx.x & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  Pair *seg = lds[wv];
   unsigned nq = 0, nlong = 0, nsplit = 0;
   for (int j = 0; j < kNBucket; ++j) {
     nq += w.ctl->hist[j];
     if (j >= w.qs.long_bucket) nlong += w.ctl->hist[j];
     if (j >= w.qs.short_bucket) nsplit += w.ctl->hist[j];
   }
-  const unsigned qchunk = (unsigned)w.qs.chunk, qschunk = (unsigned)w.qs.short_chunk;
-  const unsigned nwave = gridDim.x * (kBlock / 64);
-  const unsigned wid = blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6);
-  bool first = MAM4X_STATIC_FIRST != 0;
-  const int lane = threadIdx.x & 63;
-  const long n = w.ncell;
-  unsigned cbeg = 0, cend = 0;  // the wave's current chunk (wave-uniform)
-  bool lexhausted = false, exhausted = false;
-  bool active = false;
-  int cell = 0;
-  int emin = 0;  // the cell's dev::soa_fast_exact record
-  dev::SoaState<double> s;
+  const unsigned wid = blockIdx.x * kWaves + wv;
+  Claims cl;
+  cl.nq = nq;
+  cl.nsplit = w.quad ? nq : nsplit;
+  cl.chunk = (unsigned)w.qs.chunk;
+  cl.short_chunk = (unsigned)w.qs.short_chunk;
+  cl.ctl = w.ctl;
+  cl.lane = lane;
+  cl.init(wid, gridDim.x * kWaves);
+  if (wid * cl.chunk < nlong) __builtin_amdgcn_s_setprio(2);
+  // segment in registers (ncur records), queue entries of the one after (nnxt)
+  Staged st;
+  unsigned b, e;
+  cl.next(b, e);
+  unsigned ncur = e - b, nnxt = 0;
+  if (ncur) {
+    st.ids(w.queue, b, e, lane);
+    st.records(w.ws, lane);
+    cl.next(b, e);
+    nnxt = e - b;
+    if (nnxt) st.ids(w.queue, b, e, lane);
+  }
+  unsigned pos = 0, cnt = 0;  // the LDS segment: records pos..cnt-1 are left
+  auto advance = [&]() {      // the next segment into LDS, its successors on their way
+    st.put(seg, lane);
+    __builtin_amdgcn_wave_barrier();
+    pos = 0;
+    cnt = ncur;
+    ncur = nnxt;
+    if (ncur) {
+      st.records(w.ws, lane);
+      cl.next(b, e);
+      nnxt = e - b;
+      if (nnxt) st.ids(w.queue, b, e, lane);
+    }
+  };
   unsigned long long niter = 0;
-  while (true) {
-    const unsigned long long need = __ballot(!active);
-    if (need && cbeg == cend && !exhausted) {
-      // long part: the first chunk of every wave is assigned statically
-      // (chunk wid), later ones through the counter; then the short part
-      unsigned b0 = nsplit, e0 = nsplit;
-      if (first) {
-        first = false;
-        b0 = wid * qchunk;
-      } else if (!lexhausted) {
-        if (lane == 0) b0 = atomicAdd(&w.ctl->head, qchunk);
-        b0 = (MAM4X_STATIC_FIRST ? nwave * qchunk : 0u) +
-             __builtin_amdgcn_readfirstlane(b0);
-      }
-      if (b0 < nsplit) {
-        e0 = min(b0 + qchunk, nsplit);
-      } else {
-        lexhausted = true;
-        if (lane == 0) b0 = atomicAdd(&w.ctl->shead, qschunk);
-        b0 = nsplit + __builtin_amdgcn_readfirstlane(b0);
-        e0 = min(b0 + qschunk, nq);
-      }
-      if (MAM4X_SOA_PRIO && b0 < nlong) __builtin_amdgcn_s_setprio(2);
-      if (b0 >= nq) {
-        exhausted = true;
-      } else {
-        cbeg = b0;
-        cend = e0;
-      }
-    }
-    if (need && cbeg < cend) {
-      const unsigned rank = (unsigned)__popcll(need & ((1ull << lane) - 1ull));
-      const unsigned avail = cend - cbeg;
-      if (!active && rank < avail) {
-        cell = w.queue[cbeg + rank];
-        dev::SoaIn<double> in;
-        ws_load_in(w.ws, n, cell, in);
-        dev::soa_init(s, in);
-        emin = dev::soa_fast_ok(s, w.dtfull) ? 0 : dev::kSoaExpFail;
-        active = true;
-      }
-      cbeg += min((unsigned)__popcll(need), avail);
-    }
-    if (!__any(active)) break;
-    if (active) {
-      emin = min(emin, dev::soa_state_exp(s));
-      if (!dev::soa_tick<true>(s, w.dtfull)) {
-        // flags in the cell's bucket byte (buckets are < kIeee; the set-up
-        // kernel rewrites it every step)
-        if (emin < dev::kSoaExpMin) {
-          // inputs left untouched for soa_ieee_kernel
-          w.bucket[cell] = (unsigned char)(w.bucket[cell] | kIeee);
-        } else {
-          w.ws[W_G * n + cell] = s.g;
-#pragma unroll
-          for (int m = 0; m < 4; ++m) w.ws[(W_A + m) * n + cell] = s.a[m];
-          w.ws[W_GAVG * n + cell] = dev::soa_gavg(s);
-          niter += (unsigned long long)s.niter;
-          // the loop stopped at its cap
-          if (s.niter > 1000) w.bucket[cell] = (unsigned char)(w.bucket[cell] | kCapped);
+  int cell = -1;  // the lane's (QUAD: the four lanes') cell, -1: none
+  dev::SoaRun<1> q;
+  if (!w.quad) {
+    dev::SoaRun<4> s;
+    s.run = false;
+    while (true) {
+      const unsigned long long need = __ballot(!s.run);
+      const int nneed = __popcll(need);
+      if (nneed >= kRefill) {
+        if (!s.run && cell >= 0) {  // a finished cell
+          if (soa_done(w, cell, s.niter, s.low)) {
+            ws_store_out(w.ws, cell, s.g, s.a, soa_mean(s.avg, s.dtsum));
+            niter += (unsigned long long)s.niter;
+          }
+          cell = -1;
         }
-        active = false;
+        if (pos == cnt && ncur) advance();
+        const unsigned avail = cnt - pos;
+        if (avail) {
+          const unsigned rank = (unsigned)__popcll(need & ((1ull << lane) - 1ull));
+          if (!s.run && rank < avail) {
+            const int r = (int)(pos + rank);
+            const Pair p0 = seg_pair(seg, r, 0), p1 = seg_pair(seg, r, 1),
+                       p2 = seg_pair(seg, r, 2), p3 = seg_pair(seg, r, 3),
+                       p4 = seg_pair(seg, r, 4), p5 = seg_pair(seg, r, 5),
+                       p6 = seg_pair(seg, r, 6);
+            cell = seg_cell(seg, r);
+            const dev::SoaIn<double> in = {p0.x, {p0.y, p1.x, p1.y, p2.x}, {p3.x, p3.y, p4.x, p4.y},
+                                           {p5.x, p5.y, p6.x, p6.y}, p2.y};
+            dev::soa_run_init(s, in, w.dtfull);
+          }
+          pos += min((unsigned)nneed, avail);
+        } else if (nneed >= 64 - kQuadLanes) {
+          break;  // the queue is empty
+        }
+      }
+      if (s.run) dev::soa_run_tick(s, w.dtfull);
+    }
+    // what is left goes on in QUAD form: cells 0..15 to lanes 0..3, 4..7, ...
+    const unsigned long long left = __ballot(s.run);
+    double *x = reinterpret_cast<double *>(seg);
+    constexpr int kX = 19;
+    if (s.run) {
+      double *y = x + kX * __popcll(left & ((1ull << lane) - 1ull));
+#pragma unroll
+      for (int m = 0; m < 4; ++m) {
+        y[m] = s.a[m];
+        y[4 + m] = s.uk[m];
+        y[8 + m] = s.aopoa[m];
+      }
+      y[12] = s.g;
+      y[13] = s.g0;
+      y[14] = s.tcur;
+      y[15] = s.avg;
+      y[16] = s.dtsum;
+      y[17] = __hiloint2double(s.niter, cell);
+      y[18] = __hiloint2double(0, (int)s.low);
+    }
+    __builtin_amdgcn_wave_barrier();
+    cell = -1;
+    if ((lane >> 2) < __popcll(left)) {
+      const double *y = x + kX * (lane >> 2);
+      const int m = lane & 3;
+      q.a[0] = y[m];
+      q.uk[0] = y[4 + m];
+      q.aopoa[0] = y[8 + m];
+      q.g = y[12];
+      q.g0 = y[13];
+      q.tcur = y[14];
+      q.avg = y[15];
+      q.dtsum = y[16];
+      cell = __double2loint(y[17]);
+      q.niter = __double2hiint(y[17]);
+      q.low = (unsigned)__double2loint(y[18]);
+      q.run = true;
+    }
+    __builtin_amdgcn_wave_barrier();
+  }
+  constexpr unsigned long long kLead = 0x1111111111111111ull;  // the fours' first lanes
+  if (cell < 0) q.run = false;
+  while (true) {
+    const unsigned long long need = __ballot(!q.run) & kLead;
+    const int nneed = __popcll(need);
+    if (nneed) {
+      if (!q.run && cell >= 0) {  // a finished cell: its four lanes end together
+        unsigned low = min(q.low, (unsigned)__shfl_xor((int)q.low, 1, 64));
+        low = min(low, (unsigned)__shfl_xor((int)low, 2, 64));
+        double *o = w.ws + (long)cell * W_REC;
+        const int m = lane & 3;
+        if (low >= dev::kSoaLowMin) o[W_A + m] = q.a[0];
+        if (m == 0 && soa_done(w, cell, q.niter, low)) {
+          o[W_G] = q.g;
+          o[W_GAVG] = soa_mean(q.avg, q.dtsum);
+          niter += (unsigned long long)q.niter;
+        }
+        cell = -1;
+      }
+      if (pos == cnt && ncur) advance();
+      const unsigned avail = cnt - pos;
+      if (avail) {
+        const unsigned rank = (unsigned)__popcll(need & ((1ull << (lane & ~3)) - 1ull));
+        if (!q.run && rank < avail) {
+          const int r = (int)(pos + rank), m = lane & 3;
+          cell = seg_cell(seg, r);
+          const bool okc =
+              dev::soa_run_cell(q, seg_value(seg, r, W_G), seg_value(seg, r, W_G0), w.dtfull);
+          const bool okm =
+              dev::soa_run_mode(q, 0, seg_value(seg, r, W_A + m), seg_value(seg, r, W_UPTK + m),
+                                seg_value(seg, r, W_AOPOA + m), false);
+          q.low = okc && okm ? 0xffffffffu : 0u;
+        }
+        pos += min((unsigned)nneed, avail);
+      } else if (nneed == kQuadLanes) {
+        break;
       }
     }
+    if (q.run) dev::soa_run_tick(q, w.dtfull);
   }
   add_stats(stats, niter);
 }
@@ -442,17 +678,13 @@ __global__ void __launch_bounds__(kBlock) soa_ieee_kernel(Work w) {
   if (c < w.ncell) {
     const unsigned char b = w.bucket[c];
     if (b != kNoSoa && (b & kIeee)) {
-      const long n = w.ncell;
       dev::SoaIn<double> in;
-      ws_load_in(w.ws, n, c, in);
+      ws_load_in(w.ws, c, in);
       dev::SoaState<double> s;
       dev::soa_init(s, in);
       while (dev::soa_tick<false>(s, w.dtfull)) {
       }
-      w.ws[W_G * n + c] = s.g;
-#pragma unroll
-      for (int m = 0; m < 4; ++m) w.ws[(W_A + m) * n + c] = s.a[m];
-      w.ws[W_GAVG * n + c] = dev::soa_gavg(s);
+      ws_store_out(w.ws, c, s.g, s.a, dev::soa_gavg(s));
       niter = (unsigned long long)s.niter;
       if (s.niter > 1000) w.bucket[c] = (unsigned char)(b | kCapped);
     }
@@ -483,13 +715,13 @@ __global__ void __launch_bounds__(kBlock) chain_post_kernel(Src src, Work w) {
     dev::clear_build<P>(a, off, X, S, G);
     double uptk[4] = {0, 0, 0, 0}, sa[4] = {0, 0, 0, 0}, sg = 0.0, sgavg = 0.0;
     if (a.cfg.do_cond) {
-      const long n = w.ncell;
-      sg = w.ws[W_G * n + g];
-      sgavg = w.ws[W_GAVG * n + g];
+      const double *rec = w.ws + g * W_REC;
+      sg = rec[W_G];
+      sgavg = rec[W_GAVG];
 #pragma unroll
       for (int m = 0; m < 4; ++m) {
-        sa[m] = w.ws[(W_A + m) * n + g];
-        uptk[m] = w.ws[(W_UPTK + m) * n + g];
+        sa[m] = rec[W_A + m];
+        uptk[m] = rec[W_UPTK + m];
       }
     }
     dev::clear_post<P>(*a.K, a.cfg, a.dt, X.T, X.p, X.z, X.pblh, X.rh_clear, X.dga, X.dgw, X.wd,
@@ -643,7 +875,7 @@ __global__ void __launch_bounds__(kBlock) soa_log_kernel(AdjWork g) {
       if (!active && rank < avail) {
         cell = g.queue[cbeg + rank];
         dev::SoaIn<double> in;
-        ws_load_in(g.ws, n, cell, in);
+        ws_load_in(g.ws, cell, in);
         dev::soa_init(s, in);
         active = true;
       }
@@ -708,7 +940,7 @@ struct SoaRev {
     cell = c;
     const long n = g.ncell;
     dev::SoaIn<double> in;
-    ws_load_in(g.ws, n, c, in);
+    ws_load_in(g.ws, c, in);
     dev::soa_init(k, in);
     const double *pl = g.pb + (long)kPbSoa * n + c;
     double a_b[4];
@@ -826,7 +1058,7 @@ __global__ void __launch_bounds__(kBlock) adj_post_kernel(ChainArgs a, AdjWork g
   dev::ClearGas<double> G0;
   dev::clear_build<Fp64>(a, off, X, S0, G0);
   dev::SoaIn<double> in;
-  ws_load_in(g.ws, n, c, in);
+  ws_load_in(g.ws, c, in);
   double sa[4];
 #pragma unroll
   for (int m = 0; m < 4; ++m) sa[m] = g.res[(R_A + m) * n + c];
@@ -1828,12 +2060,12 @@ static void launch_order(bool pre, unsigned grid, hipStream_t s, const OneDomain
 }
 
 // Device memory of the allocation-free step (mam4x_compute_tendencies_noalloc):
-// the work-queue workspace for up to kScratchCells cells -- W_NPLANE planes of
-// doubles, the queue, the cost buckets -- and the queue counters.  Every GPU the
+// the work-queue workspace for up to kScratchCells cells -- W_REC doubles
+// a cell, the queue, the cost buckets -- and the queue counters.  Every GPU the
 // library runs on holds one copy (117 B per cell: 61.3 MB) until the process
 // ends; every call on a GPU shares it, so calls that overlap on one GPU race.
 static constexpr long kScratchCells = MAM4X_NOALLOC_MAX_CELLS;
-static constexpr size_t kScratchWsBytes = sizeof(double) * W_NPLANE * kScratchCells;
+static constexpr size_t kScratchWsBytes = sizeof(double) * W_REC * kScratchCells;
 static constexpr size_t kScratchQueueOff = kScratchWsBytes;
 static constexpr size_t kScratchBucketOff = kScratchQueueOff + sizeof(int) * kScratchCells;
 static constexpr size_t kScratchCtlOff =
@@ -1871,7 +2103,11 @@ struct mam4x_handle_s {
   unsigned long long *d_count = nullptr;  // validate counter
   unsigned long long *d_stats = nullptr;  // SOA sub-steps since the last read
   bool stats = false;
-  // work-queue schedule: workspace for up to `cap` cells (grown on demand)
+  // the buffers below d_consts to ctl, and a workspace for kFirstCells cells
+  unsigned char *base = nullptr, *first = nullptr;
+  // work-queue schedule: workspace for up to `cap` cells (grown on demand),
+  // `work` its own allocation, or NULL while it is `first` (in `base`)
+  unsigned char *work = nullptr;
   long cap = 0;
   double *ws = nullptr;
   unsigned char *bucket = nullptr;
@@ -1900,9 +2136,7 @@ struct mam4x_handle_s {
   std::string err;
 };
 
-// cells below which the fused one-lane-per-cell kernel is used by
-// MAM4X_SCHED_AUTO: small domains do not fill the chip with persistent waves
-// and pay four launches for little divergence saving
+// cells below which MAM4X_SCHED_AUTO takes the fused kernel for ntsubstep > 1
 static constexpr long kFusedBelow = 16384;
 
 static void destroy_events(mam4x_handle h) {
@@ -1913,14 +2147,36 @@ static void destroy_events(mam4x_handle h) {
   h->pool.clear();
 }
 
-static void free_work(mam4x_handle h) {
-  if (h->ws) (void)hipFree(h->ws);
-  if (h->bucket) (void)hipFree(h->bucket);
-  if (h->queue) (void)hipFree(h->queue);
-  h->ws = nullptr;
-  h->bucket = nullptr;
-  h->queue = nullptr;
-  h->cap = 0;
+// A workspace of ncell cells: the records, the queue, the cost buckets.
+static constexpr long kFirstCells = 16384;
+static constexpr size_t work_bytes(long ncell) {
+  return (sizeof(double) * W_REC + sizeof(int) + 1) * (size_t)ncell;
+}
+static void set_work(mam4x_handle h, unsigned char *p, long ncell) {
+  h->ws = reinterpret_cast<double *>(p);
+  h->queue = reinterpret_cast<int *>(p + sizeof(double) * W_REC * ncell);
+  h->bucket = p + (sizeof(double) * W_REC + sizeof(int)) * ncell;
+  h->cap = ncell;
+}
+
+// Cells up to which soa_queue_kernel starts in its QUAD form.  Up to there the
+// longest chains set its time and the chip has issue slots to spare; beyond,
+// the work does.  One-lane against QUAD form, ms per step at 72 levels: 1000
+// columns 0.736 / 0.653, 2000 0.823 / 0.797, 2701 0.842 / 0.868, 5400 1.150 /
+// 1.426.
+static constexpr long kQuadCells = 163840;
+
+// soa_queue_kernel over w.ncell cells: its form, its claims (16 cells fill a
+// wave in QUAD form) and its grid, no larger than its claims need
+static void launch_soa_queue(mam4x_handle h, Work w, hipStream_t s) {
+  w.quad = w.ncell <= kQuadCells;
+  if (w.quad && !h->cfg.soa_chunk) w.qs.chunk = kQuadLanes;
+  // a wave's first claim starts at its index times the claim, in 32 bits
+  w.qs.chunk = std::min(w.qs.chunk, 1 << 18);
+  const long claim = w.quad ? w.qs.chunk : std::min(w.qs.chunk, w.qs.short_chunk);
+  const long waves = (w.ncell + claim - 1) / claim;
+  const unsigned grid = (unsigned)std::min<long>(h->soa_grid, (waves + kWaves - 1) / kWaves);
+  hipLaunchKernelGGL(soa_queue_kernel, dim3(grid), dim3(kBlock), 0, s, w, w.stats);
 }
 
 static int fail(mam4x_handle h, int code, const std::string &msg) {
@@ -1935,21 +2191,24 @@ static int fail(mam4x_handle h, int code, const std::string &msg) {
       return fail((h), MAM4X_ERR_HIP, std::string(#expr) + ": " + hipGetErrorString(e_)); \
   } while (0)
 
-// Workspace for ncell cells.  Growing frees the old buffers only after the
-// stream has drained, since earlier launches may still use them.
+// Workspace for ncell cells.  Growing frees an earlier allocation only after
+// the stream has drained, since earlier launches may still use it; the first
+// workspace stays with the handle.
 static int reserve_work(mam4x_handle h, long ncell, hipStream_t s) {
   if (ncell <= h->cap) return MAM4X_OK;
-  if (h->cap) HIP_TRY(h, hipStreamSynchronize(s));
-  free_work(h);
-  if (hipMalloc(&h->ws, sizeof(double) * W_NPLANE * ncell) != hipSuccess ||
-      hipMalloc(&h->bucket, (size_t)ncell) != hipSuccess ||
-      hipMalloc(&h->queue, sizeof(int) * ncell) != hipSuccess) {
+  if (h->work) {
+    HIP_TRY(h, hipStreamSynchronize(s));
+    (void)hipFree(h->work);
+    h->work = nullptr;
+    set_work(h, h->first, kFirstCells);
+  }
+  if (hipMalloc(&h->work, work_bytes(ncell)) != hipSuccess) {
     (void)hipGetLastError();
-    free_work(h);
+    h->work = nullptr;
     return fail(h, MAM4X_ERR_NOMEM, "workspace allocation failed (" +
                 std::to_string(ncell) + " cells)");
   }
-  h->cap = ncell;
+  set_work(h, h->work, ncell);
   return MAM4X_OK;
 }
 
@@ -2059,11 +2318,11 @@ static bool config_ok(const mam4x_config &c) {
 }
 
 // Resident blocks of the persistent SOA kernel per CU when the
-// configuration leaves it at 0.  Measured on 21,600 x 72, chained steps from
-// the seeded state: 3 blocks (12 waves per CU) 2.842 ms per step against
-// 2.896 with as many as fit (4) over steps 1-10, and 2.611 against 2.605
-// over steps 11-20.
-constexpr int kSoaBlocksDefault = 3;
+// configuration leaves it at 0.  Two waves a SIMD keep its issue port busy, and
+// a third only slows the longest chains.  2 against 3 blocks, ms per step:
+// 2,701 x 72 0.957 / 1.030, 21,600 x 72 3.447 / 3.516, 43,200 x 128 9.38 /
+// 9.55.
+constexpr int kSoaBlocksDefault = 2;
 
 // Resident blocks per CU of the reverse sweep's SOA log kernel (its replay
 // kernel runs one wave per log wave).  Measured on the 21,600 x 72 sweep of
@@ -2114,14 +2373,23 @@ int mam4x_create(const mam4x_config *config, mam4x_handle *out) {
   if (scratch_address(h->device, &h->scratch) != MAM4X_OK) h->scratch = nullptr;
   ChainConsts k;
   chain_consts_init(&k);
-  if (hipMalloc(&h->d_consts, sizeof(ChainConsts)) != hipSuccess ||
-      hipMalloc(&h->d_count, sizeof(unsigned long long)) != hipSuccess ||
-      hipMalloc(&h->d_stats, sizeof(unsigned long long)) != hipSuccess ||
-      hipMalloc(&h->ctl, sizeof(QueueCtl)) != hipSuccess) {
+  // one allocation for the small buffers and a first workspace, so that the
+  // first step of a small domain allocates nothing
+  constexpr size_t kAlign = 256, kConstBytes = (sizeof(ChainConsts) + kAlign - 1) / kAlign * kAlign,
+                   kCtlBytes = (sizeof(QueueCtl) + kAlign - 1) / kAlign * kAlign;
+  if (hipMalloc(&h->base, kConstBytes + 2 * kAlign + kCtlBytes + work_bytes(kFirstCells)) !=
+      hipSuccess) {
     (void)hipGetLastError();
     mam4x_destroy(h);
     return MAM4X_ERR_NOMEM;
   }
+  unsigned char *p = h->base;
+  h->d_consts = reinterpret_cast<ChainConsts *>(p);
+  h->d_count = reinterpret_cast<unsigned long long *>(p += kConstBytes);
+  h->d_stats = reinterpret_cast<unsigned long long *>(p += kAlign);
+  h->ctl = reinterpret_cast<QueueCtl *>(p += kAlign);
+  h->first = p + kCtlBytes;
+  set_work(h, h->first, kFirstCells);
   if (hipMemcpy(h->d_consts, &k, sizeof(k), hipMemcpyHostToDevice) != hipSuccess ||
       hipMemset(h->d_stats, 0, sizeof(unsigned long long)) != hipSuccess) {
     mam4x_destroy(h);
@@ -2133,14 +2401,9 @@ int mam4x_create(const mam4x_config *config, mam4x_handle *out) {
 
 int mam4x_destroy(mam4x_handle h) {
   if (!h) return MAM4X_ERR_ARG;
-  if (h->d_consts) (void)hipFree(h->d_consts);
-  if (h->d_count) (void)hipFree(h->d_count);
-  if (h->d_stats) (void)hipFree(h->d_stats);
-  if (h->ctl) (void)hipFree(h->ctl);
-  for (void *q : {(void *)h->adjws, (void *)h->subws, (void *)h->log_rec, (void *)h->log_tag,
+  for (void *q : {(void *)h->base, (void *)h->work, (void *)h->adjws, (void *)h->subws, (void *)h->log_rec, (void *)h->log_tag,
                   (void *)h->log_prev, (void *)h->log_wend, (void *)h->log_next})
     if (q) (void)hipFree(q);
-  free_work(h);
   destroy_events(h);
   delete h;
   return MAM4X_OK;
@@ -2359,7 +2622,7 @@ int mam4x_compute_tangent(mam4x_handle h, double t, double dt, const mam4x_input
     w.dtfull = dev::dt_sub(a.cfg, dt);
     hipLaunchKernelGGL(queue_reset_kernel, dim3(1), dim3(64), 0, s, w.ctl);
     launch_cells<Fp64>(kPre, pre, grid, s, src, w);
-    hipLaunchKernelGGL(queue_scatter_kernel, dim3(grid), dim3(kBlock), 0, s, w);
+    hipLaunchKernelGGL(queue_scatter_kernel, dim3(scatter_grid(w.ncell)), dim3(kBlock), 0, s, w);
     for (int pass = 0; pass < 2; ++pass) {
       if (multi)
         launch_order<Tangent, true>(pre, grid, s, src, w, pass);
@@ -2474,7 +2737,7 @@ int mam4x_compute_adjoint(mam4x_handle h, double t, double dt, const mam4x_input
       w.queue = h->queue;
       hipLaunchKernelGGL(queue_reset_kernel, dim3(1), dim3(64), 0, s, h->ctl);
       launch_cells<Fp64>(kPre, pre, grid, s, OneDomain{a}, w);
-      hipLaunchKernelGGL(queue_scatter_kernel, dim3(grid), dim3(kBlock), 0, s, w);
+      hipLaunchKernelGGL(queue_scatter_kernel, dim3(scatter_grid(w.ncell)), dim3(kBlock), 0, s, w);
       queue = h->queue;
       ctl = h->ctl;
       o.bucket = h->bucket;
@@ -2522,7 +2785,7 @@ int mam4x_compute_adjoint(mam4x_handle h, double t, double dt, const mam4x_input
     const OneDomain src{a};
     hipLaunchKernelGGL(queue_reset_kernel, dim3(1), dim3(64), 0, s, h->ctl);
     launch_cells<Fp64>(kPre, pre, grid, s, src, w);
-    hipLaunchKernelGGL(queue_scatter_kernel, dim3(grid), dim3(kBlock), 0, s, w);
+    hipLaunchKernelGGL(queue_scatter_kernel, dim3(scatter_grid(w.ncell)), dim3(kBlock), 0, s, w);
     HIP_TRY(h, hipGetLastError());
     AdjWork g;
     g.qs = queue_shape(h->cfg);
@@ -2778,8 +3041,13 @@ static int compute_step(mam4x_handle h, double dt, const mam4x_inputs *in,
   const long ncell = (long)in->ncol * in->nlev;
   if (ncell == 0) return out->column_budgets ? launch_budgets(h, in, out, s) : MAM4X_OK;
   const unsigned grid = (unsigned)((ncell + kBlock - 1) / kBlock);
-  bool fused = h->cfg.schedule == MAM4X_SCHED_FUSED ||
-               (h->cfg.schedule == MAM4X_SCHED_AUTO && ncell < kFusedBelow);
+  // the queue also for the smallest domains: its QUAD form halves the longest
+  // SOA chain (1 column x 72: 0.262 ms a step against 0.452 fused, 16: 0.551 /
+  // 0.867, 200: 0.573 / 1.372)
+  // (one sub-step; with more, one lane runs a cell either way)
+  const bool fused =
+      h->cfg.schedule == MAM4X_SCHED_FUSED ||
+      (h->cfg.schedule == MAM4X_SCHED_AUTO && dev::nsub(a.cfg) > 1 && ncell < kFusedBelow);
   // ntsubstep > 1: one lane runs a cell's whole step (the split phases hold
   // one sub-step), in the queue's order unless the fused schedule is chosen
   const bool multi = dev::nsub(a.cfg) > 1;
@@ -2793,7 +3061,7 @@ static int compute_step(mam4x_handle h, double dt, const mam4x_inputs *in,
   const OneDomain src{a};
   const bool queue = !fused && a.cfg.do_cond;
   if (queue && noalloc) {
-    // W_NPLANE planes of ncell doubles fit the kScratchCells-sized region
+    // ncell records fit the kScratchCells-sized region
     w.ws = reinterpret_cast<double *>(h->scratch);
     w.queue = reinterpret_cast<int *>(h->scratch + kScratchQueueOff);
     w.bucket = h->scratch + kScratchBucketOff;
@@ -2823,11 +3091,11 @@ static int compute_step(mam4x_handle h, double dt, const mam4x_inputs *in,
       launch_cells<Mixed>(kPre, pre, grid, s, src, w);
     else
       launch_cells<Fp64>(kPre, pre, grid, s, src, w);
-    hipLaunchKernelGGL(queue_scatter_kernel, dim3(grid), dim3(kBlock), 0, s, w);
+    hipLaunchKernelGGL(queue_scatter_kernel, dim3(scatter_grid(w.ncell)), dim3(kBlock), 0, s, w);
   }
   if (ev) HIP_TRY(h, hipEventRecord(ev[1], s));
   if (queue && !multi) {
-    hipLaunchKernelGGL(soa_queue_kernel, dim3(h->soa_grid), dim3(kBlock), 0, s, w, w.stats);
+    launch_soa_queue(h, w, s);
     hipLaunchKernelGGL(soa_ieee_kernel, dim3(grid), dim3(kBlock), 0, s, w);
   }
   if (ev) HIP_TRY(h, hipEventRecord(ev[2], s));
@@ -3348,12 +3616,11 @@ int mam4x_batch_create(mam4x_handle h, int nscene, const mam4x_inputs *in,
       budget_args(&in[i], &out[i], b->budgets.back());
     }
   b->fused = h->cfg.schedule == MAM4X_SCHED_FUSED ||
-             (h->cfg.schedule == MAM4X_SCHED_AUTO && b->ncell < kFusedBelow) ||
              h->cfg.ntsubstep > 1;  // the split phases hold one sub-step
   b->queue = !b->fused && args[0].cfg.do_cond != 0 && b->ncell > 0;
   if (hipMalloc(&b->d_args, sizeof(ChainArgs) * nscene) != hipSuccess ||
       hipMalloc(&b->d_blk0, sizeof(unsigned) * (nscene + 1)) != hipSuccess ||
-      (b->queue && (hipMalloc(&b->ws, sizeof(double) * W_NPLANE * b->ncell) != hipSuccess ||
+      (b->queue && (hipMalloc(&b->ws, sizeof(double) * W_REC * b->ncell) != hipSuccess ||
                     hipMalloc(&b->bucket, (size_t)b->ncell) != hipSuccess ||
                     hipMalloc(&b->wqueue, sizeof(int) * b->ncell) != hipSuccess ||
                     hipMalloc(&b->ctl, sizeof(QueueCtl)) != hipSuccess))) {
@@ -3407,8 +3674,8 @@ int mam4x_batch_run(mam4x_batch b, double t, double dt, void *stream) {
       launch_cells<Mixed>(kPre, b->pre, b->nblock, s, src, w);
     else
       launch_cells<Fp64>(kPre, b->pre, b->nblock, s, src, w);
-    hipLaunchKernelGGL(queue_scatter_kernel, dim3(b->nblock), dim3(kBlock), 0, s, w);
-    hipLaunchKernelGGL(soa_queue_kernel, dim3(h->soa_grid), dim3(kBlock), 0, s, w, w.stats);
+    hipLaunchKernelGGL(queue_scatter_kernel, dim3(scatter_grid(w.ncell)), dim3(kBlock), 0, s, w);
+    launch_soa_queue(h, w, s);
     hipLaunchKernelGGL(soa_ieee_kernel, dim3(b->nblock), dim3(kBlock), 0, s, w);
   }
   const int kind = fused ? kFused : kPost;

@@ -169,6 +169,30 @@ __host__ __device__ __forceinline__ double div_fast(double a, double b) {
 __host__ __device__ __forceinline__ F32 div_fast(F32 a, F32 b) { return a / b; }
 __host__ __device__ __forceinline__ Dual div_fast(Dual a, Dual b) { return a / b; }
 
+// ------------------------------------------------------------------ max
+// The larger of two numbers, neither of them NaN: one instruction on the GPU,
+// where the ternary form is a compare and two selects.  Of a -0 and a +0 the
+// GPU returns +0.
+__host__ __device__ __forceinline__ double vmax(double a, double b) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  double r;
+  asm("v_max_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+  return r;
+#else
+  return (a < b) ? b : a;
+#endif
+}
+// sign, exponent and the upper fraction bits
+__host__ __device__ __forceinline__ unsigned high_word(double x) {
+#if defined(__HIP__)
+  return (unsigned)__double2hiint(x);
+#else
+  unsigned long long u;
+  __builtin_memcpy(&u, &x, sizeof(u));
+  return (unsigned)(u >> 32);
+#endif
+}
+
 // ------------------------------------------------------------------ helpers
 // primal value as a double (branch decisions, integer indices, outputs)
 __host__ __device__ __forceinline__ double val(double x) { return x; }
