@@ -190,6 +190,16 @@ struct Work {
 struct OneDomain {
   ChainArgs a;
   __device__ __forceinline__ const ChainArgs &scene(long &c) const { return a; }
+  // the same, as a block that dev::again can load from again: the kernels take
+  // their source first, so it opens their argument segment
+  __device__ __forceinline__ const ChainArgs &kargs(long &c) const {
+#if defined(__HIP_DEVICE_COMPILE__)
+    return *(const ChainArgs *)(const __attribute__((address_space(4))) ChainArgs *)
+        __builtin_amdgcn_kernarg_segment_ptr();
+#else
+    return a;
+#endif
+  }
 };
 
 struct SceneBatch {
@@ -209,6 +219,7 @@ struct SceneBatch {
     c = (long)(b - blk0[lo]) * kBlock + threadIdx.x;
     return args[lo];
   }
+  __device__ __forceinline__ const ChainArgs &kargs(long &c) const { return scene(c); }
 };
 
 // cell c of the memory-order enumeration -> column and plane offset
@@ -697,7 +708,9 @@ template <bool PRE, class P, class Src>
 __global__ void __launch_bounds__(kBlock) chain_post_kernel(Src src, Work w) {
   const long g = (long)blockIdx.x * kBlock + threadIdx.x;  // workspace index
   long c = g;
-  const ChainArgs &a = src.scene(c);
+  constexpr bool KARGS = !P::diag;
+  const ChainArgs &a0 = KARGS ? src.kargs(c) : src.scene(c);
+  const ChainArgs &a = dev::again<KARGS>(a0, 1);
   if (g >= w.ncell || c >= (long)a.ncol * a.nlev) return;
   int icol;
   long off;
@@ -712,7 +725,7 @@ __global__ void __launch_bounds__(kBlock) chain_post_kernel(Src src, Work w) {
     D.zero();
   }
   if (X.cat != 1) {
-    dev::clear_build<P>(a, off, X, S, G);
+    dev::clear_build<P>(dev::again<KARGS>(a0, 2), off, X, S, G);
     double uptk[4] = {0, 0, 0, 0}, sa[4] = {0, 0, 0, 0}, sg = 0.0, sgavg = 0.0;
     if (a.cfg.do_cond) {
       const double *rec = w.ws + g * W_REC;
@@ -727,7 +740,7 @@ __global__ void __launch_bounds__(kBlock) chain_post_kernel(Src src, Work w) {
     dev::clear_post<P>(*a.K, a.cfg, a.dt, X.T, X.p, X.z, X.pblh, X.rh_clear, X.dga, X.dgw, X.wd,
                     G.g1, G.g, S, uptk, sg, sgavg, sa, &D);
   }
-  dev::cell_finish<PRE, P>(a, off, X, S, G);
+  dev::cell_finish<PRE, P, false, KARGS>(a0, off, X, S, G);
   if (a.soacap)
     a.soacap[off] = (a.cfg.do_cond && X.cat != 1 && (w.bucket[g] & kCapped)) ? 1 : 0;
 }
