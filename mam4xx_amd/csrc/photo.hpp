@@ -280,39 +280,46 @@ __host__ __device__ __forceinline__ LevelPos level_pos(const Table &t, const Sza
 // [numcolo3][numalb], xsqy [numj][nw][nt][np_xs].
 struct RowMajor {
   const double *rsf, *xs;  // xs: xsqy of the reaction
-  long s_al, s_v, s_s, s_z, s_w, x_p, x_t, x_w;
+  long s_v, s_s, s_z, s_w, x_t, x_w;
   __host__ __device__ RowMajor(const Table &t) {
     rsf = t.rsf_tab;
-    s_al = 1;
     s_v = t.numalb;
     s_s = (long)t.numcolo3 * s_v;
     s_z = (long)t.numsza * s_s;
     s_w = (long)t.nump * s_z;
-    x_p = 1;
     x_t = t.np_xs;
     x_w = (long)t.nt * x_t;
     xs = t.xsqy + (long)t.ind * t.nw * x_w;
   }
 };
 
-template <class Ix>
-__host__ __device__ __forceinline__ double corner_sum(const Corners &c, const Ix &x,
+// two table neighbours in one load
+struct __attribute__((aligned(8))) Two {
+  double x, y;
+};
+__host__ __device__ __forceinline__ Two two(const double *p) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return *reinterpret_cast<const Two *>(p);
+#else
+  return Two{p[0], p[1]};
+#endif
+}
+
+__host__ __device__ __forceinline__ double corner_sum(const Corners &c, const RowMajor &x,
                                                       const double *r) {
-  return c.w000 * r[0] + c.w001 * r[x.s_al] + c.w010 * r[x.s_v] + c.w011 * r[x.s_v + x.s_al] +
-         c.w100 * r[x.s_s] + c.w101 * r[x.s_s + x.s_al] + c.w110 * r[x.s_s + x.s_v] +
-         c.w111 * r[x.s_s + x.s_v + x.s_al];
+  const Two v0 = two(r), v1 = two(r + x.s_v), v2 = two(r + x.s_s), v3 = two(r + x.s_s + x.s_v);
+  return c.w000 * v0.x + c.w001 * v0.y + c.w010 * v1.x + c.w011 * v1.y + c.w100 * v2.x +
+         c.w101 * v2.y + c.w110 * v3.x + c.w111 * v3.y;
 }
 
 // one wavelength's term of jlong's sum: the cross section times the source
 // function interpolated in zenith angle, ozone ratio, albedo and pressure
-template <class Ix>
-__host__ __device__ __forceinline__ double wn_term(const Table &t, const Ix &x,
+__host__ __device__ __forceinline__ double wn_term(const Table &t, const RowMajor &x,
                                                    const LevelPos &q, const Corners &cl,
                                                    const Corners &cu, int wn) {
-  const double *rl = x.rsf + q.pind * x.s_z + q.is * x.s_s + q.ratl * x.s_v + q.ial * x.s_al +
-                     wn * x.s_w;
-  const double *ru = x.rsf + (q.pind - 1) * x.s_z + q.is * x.s_s + q.ratu * x.s_v +
-                     q.ial * x.s_al + wn * x.s_w;
+  const double *rl = x.rsf + q.pind * x.s_z + q.is * x.s_s + q.ratl * x.s_v + q.ial + wn * x.s_w;
+  const double *ru =
+      x.rsf + (q.pind - 1) * x.s_z + q.is * x.s_s + q.ratu * x.s_v + q.ial + wn * x.s_w;
   const double psum_l = corner_sum(cl, x, rl);
   const double psum_u = corner_sum(cu, x, ru);
   const double rsf = (psum_l + q.wght1 * (psum_u - psum_l)) * t.etfphot[wn];
@@ -321,26 +328,28 @@ __host__ __device__ __forceinline__ double wn_term(const Table &t, const Ix &x,
   if (q.pcase == 0) {
     xswk = xr[0];
   } else if (q.pcase == 1) {
-    xswk = xr[(t.np_xs - 1) * x.x_p];
+    xswk = xr[t.np_xs - 1];
   } else {
-    const double x0 = xr[q.pndx * x.x_p], x1 = xr[(q.pndx + 1) * x.x_p];
-    xswk = x0 + q.delp * (x1 - x0);
+    const Two v = two(xr + q.pndx);
+    xswk = v.x + q.delp * (v.y - v.x);
   }
   return xswk * rsf;
 }
 
 // photolysis rate of reaction t.ind at one level, the wavelengths summed in
 // order (interpolate_rsf + jlong), from the tables as given
-__host__ __device__ __forceinline__ double level_rate(const Table &t, const SzaPos &s,
-                                                      double alb_in, double p_in, double t_in,
-                                                      double colo3_in) {
-  const LevelPos q = level_pos(t, s, alb_in, p_in, t_in, colo3_in);
+__host__ __device__ __forceinline__ double level_rate(const Table &t, const LevelPos &q) {
   const Corners cl = corners(q.dels0, q.wrk0, q.d1l, q.d2);
   const Corners cu = corners(q.dels0, q.wrk0, q.d1u, q.d2);
   const RowMajor x(t);
   double suma = 0.0;
   for (int wn = 0; wn < t.nw; ++wn) suma += wn_term(t, x, q, cl, cu, wn);
   return suma;
+}
+__host__ __device__ __forceinline__ double level_rate(const Table &t, const SzaPos &s,
+                                                      double alb_in, double p_in, double t_in,
+                                                      double colo3_in) {
+  return level_rate(t, level_pos(t, s, alb_in, p_in, t_in, colo3_in));
 }
 
 // table_photo's update of one level's rate
