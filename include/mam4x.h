@@ -119,7 +119,7 @@ typedef struct mam4x_config {
   int precision; /* MAM4X_PREC_*                                          */
   int schedule;  /* MAM4X_SCHED_*                                         */
   int soa_blocks_per_cu; /* persistent SOA kernel: resident blocks per CU,
-                            at most as many as fit; 0 = 3 (performance
+                            at most as many as fit; 0 = 2 (performance
                             only)                                        */
   int ntsubstep; /* condensation sub-steps per step, 1..MAM4X_MAX_NTSUBSTEP
                     (0 is taken as 1).  The reference fixes 1
@@ -135,7 +135,8 @@ typedef struct mam4x_config {
                     (:1446-1455).  n > 1 runs the one-lane-per-cell schedule. */
   /* Performance only (results are identical; 0 = default):
    *  soa_chunk        queue entries a wave takes per refill from the long
-   *                   part of the SOA work queue (default 64);
+   *                   part of the SOA work queue (default 64, or
+   *                   16 where four lanes take a cell);
    *  soa_short_chunk  the same for the short part (default 256);
    *  soa_short_bucket first cost bucket of the long part, 1..24 (default 10:
    *                   predicted <= ~30 sub-steps go to the short part);
