@@ -229,7 +229,7 @@ __device__ __forceinline__ num::Dual soa_term(bool skip, num::Dual x) {
 // One pass of the while loop (gasaerexch_soaexch.hpp:170-335).  Returns false
 // once the loop has ended (time reached or 1000 sub-steps taken).
 //
-// FAST divides with num::div_fast (reciprocal, Markstein
+// FAST divides with num::div_fast (reciprocal, Newton steps, Markstein
 // correction: IEEE's quotient wherever numerators are 0 or at least 2^-968,
 // quotients normal and divisors in range); otherwise each quotient is the
 // IEEE a / b.  soa_fast_exact below states when every FAST quotient of a

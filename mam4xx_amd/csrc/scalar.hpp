@@ -127,31 +127,35 @@ __host__ __device__ __forceinline__ Dual fabs(Dual a) { return a.v < 0 ? -a : a;
 __host__ __device__ __forceinline__ Dual round(Dual a) { return Dual(::round(a.v), 0.0); }
 
 // ------------------------------------------------------------------ division
-// Correctly rounded FP64 division without the range scaling and special-case
-// fix-up of the general IEEE sequence: the reciprocal to the last place, then
-// q + r (a - b q) (Markstein).  It equals a / b whenever a, b and a/b are
-// normal numbers away from the ends of the exponent range (|a| >= 2^-968,
-// 2^-1021 < |b| < 2^1021, |a/b| >= 2^-1021); a +0 numerator gives +0, a -0
-// numerator +0 as well (IEEE: -0).  Below 2^-968 the residual a - b q is not
-// representable and the quotient can be one unit in the last place off; b = 0
-// or inf gives NaN.  Callers use it only where they know the operands to be in
-// range (the SOA sub-step, whose loop checks that it is: soa_fast_exact in
-// chain_device.hpp).
+// The compiler's a / b without the range scaling and special-case fix-up of its
+// general sequence: reciprocal, two Newton steps, then
+// q + r (a - b q) (Markstein).  These are the same operations the general
+// sequence performs when its scaling is the identity, which holds whenever a,
+// b and a/b are normal numbers away from the ends of the exponent range
+// (|a| >= 2^-968, 2^-1021 < |b| < 2^1021, |a/b| >= 2^-1021); a +0 numerator
+// gives +0, a -0 numerator +0 as well (IEEE: -0).  Below 2^-968 the residual
+// a - b q is not representable and the quotient can be one unit in the last
+// place off; b = 0 or inf gives NaN.  Callers use it only where they know
+// the operands to be in range (the SOA sub-step, whose loop checks that it
+// is: soa_fast_exact in chain_device.hpp).
 //
-// rcp(b): the hardware's seed r has 24 bits, so with e = 1 - b r one step of
-// third order, r + r (e + e^2), leaves a relative error of e^3 ~ 2^-72 before
-// its rounding: three multiply-adds, where two Newton steps take four.  Over
-// 2^26 divisors the seed was within 2^-24.37 and r within 0.50000008 units in
-// the last place (Newton: 0.5; 3 of the r differ); no quotient differs
-// (tests/test_gpu_division.py).  The SOA sub-step takes 18 reciprocals: its
-// kernel 2.27 -> 2.13 ms on 21,600 x 72.  div_r(a, b, r) is the quotient from it, so a
-// divisor used more than once is inverted once: div_fast(a, b) = div_r(a, b,
-// rcp(b)).  Host builds divide with a / b.
+// rcp(b) is the reciprocal with its two Newton steps and div_r(a, b, r) the
+// quotient from it, so a divisor used more than once is inverted once:
+// div_fast(a, b) = div_r(a, b, rcp(b)).  Host builds divide with a / b.
+// One step of third order, r + r (e + e^2), would take a multiply-add less
+// (21,600 x 72: 3.26 against 3.42 ms a step), but it rounds one of some 2^24
+// reciprocals wrong (1 / 0x1.0780514b0b125p+61), which the reverse sweep takes
+// without a correction, and its quotients are no longer the general sequence's
+// where that is itself a last place off IEEE's (divisors such as
+// 0x1.ffffffffffffdp+0: 3 of 131,072 constructed pairs;
+// tests/test_gpu_division.py).
 __host__ __device__ __forceinline__ double rcp(double b) {
 #if defined(__HIP_DEVICE_COMPILE__)
-  const double r = __builtin_amdgcn_rcp(b);
-  const double e = __builtin_fma(-b, r, 1.0);
-  return __builtin_fma(r, __builtin_fma(e, e, e), r);
+  double r = __builtin_amdgcn_rcp(b);
+  double e = __builtin_fma(-b, r, 1.0);
+  r = __builtin_fma(r, e, r);
+  e = __builtin_fma(-b, r, 1.0);
+  return __builtin_fma(r, e, r);
 #else
   return 1.0 / b;
 #endif

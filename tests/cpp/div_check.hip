@@ -47,7 +47,26 @@ __global__ void div_check_kernel(long n, unsigned long long seed, int tiny,
   }
 }
 
+// rows of n: num::rcp(b), num::div_fast(a, b), and the compiler's 1 / b, a / b
+__global__ void div_arrays_kernel(long n, const double *a, const double *b, double *out) {
+  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  out[i] = mam4x::num::rcp(b[i]);
+  out[n + i] = mam4x::num::div_fast(a[i], b[i]);
+  out[2 * n + i] = 1.0 / b[i];
+  out[3 * n + i] = a[i] / b[i];
+}
+
 }  // namespace
+
+// Reciprocals and quotients of n operand pairs, out 4 n values, all in device
+// memory; 0, or -1 on a HIP error.
+extern "C" int div_arrays(long n, const double *a, const double *b, double *out) {
+  if (n <= 0) return n == 0 ? 0 : -1;
+  hipLaunchKernelGGL(div_arrays_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, 0, n, a,
+                     b, out);
+  return hipGetLastError() == hipSuccess && hipDeviceSynchronize() == hipSuccess ? 0 : -1;
+}
 
 // Returns the number of operand pairs (out of n) inside the exact range where
 // the two quotients differ in any bit; the first such pair goes to
