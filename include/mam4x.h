@@ -137,7 +137,8 @@ typedef struct mam4x_config {
    *  soa_chunk        queue entries a wave takes per refill from the long
    *                   part of the SOA work queue (default 64, or
    *                   16 where four lanes take a cell);
-   *  soa_short_chunk  the same for the short part (default 256);
+   *  soa_short_chunk  the same for the short part (default 256); both up to
+   *                   2^20, taken as 2^18 above that;
    *  soa_short_bucket first cost bucket of the long part, 1..24 (default 10:
    *                   predicted <= ~30 sub-steps go to the short part);
    *  levels_per_wave  1, 2, 4 or 8: the per-cell kernels give each wave a

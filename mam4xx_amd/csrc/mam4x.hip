@@ -39,6 +39,7 @@
 #include "gas_chem.hpp"
 #include "linoz.hpp"
 #include "photo.hpp"
+#include "queue_claims.hpp"
 #include "sethet.hpp"
 #include "setsox.hpp"
 #include "water_uptake.hpp"
@@ -48,31 +49,12 @@ using namespace mam4x;
 namespace {
 
 constexpr int kBlock = 256;
-constexpr int kNBucket = 24;  // half-octave cost buckets: 2 log2(1 + predicted sub-steps)
-#ifndef MAM4X_QUEUE_CHUNK
-#define MAM4X_QUEUE_CHUNK 64
-#endif
-constexpr int kChunk = MAM4X_QUEUE_CHUNK;  // default queue entries a wave takes per refill
 // Waves whose first chunk comes from buckets >= kLongBucket (predicted >= ~180
 // sub-steps) raise their issue priority: a cell's sub-steps are a serial
 // chain, so the longest cells set the kernel's critical path and should not
 // yield issue slots to the bulk.
 #ifndef MAM4X_SOA_PRIO
 #define MAM4X_SOA_PRIO 1
-#endif
-constexpr int kLongBucket = 15;
-// Refills cost a device-scope atomic on a queue counter, and those atomics
-// serialise across the device (tens of ns each), so the kernel keeps their
-// number down: every wave's first chunk is assigned statically (chunk = wave
-// index: the longest cells go to the first-dispatched, oldest waves), and the
-// cells of buckets < kShortBucket (predicted <= ~30 sub-steps) form a second
-// part of the queue taken kShortChunk at a time -- holding a few short cells
-// back in a busy wave costs little.
-#ifndef MAM4X_SHORT_BUCKET
-#define MAM4X_SHORT_BUCKET 10
-#endif
-#ifndef MAM4X_SHORT_CHUNK
-#define MAM4X_SHORT_CHUNK 256
 #endif
 #ifndef MAM4X_STATIC_FIRST
 #define MAM4X_STATIC_FIRST 1
@@ -85,8 +67,6 @@ constexpr int kLongBucket = 15;
 #ifndef MAM4X_ADJ_PRE_WAVES
 #define MAM4X_ADJ_PRE_WAVES 2
 #endif
-constexpr int kShortBucket = MAM4X_SHORT_BUCKET;
-constexpr int kShortChunk = MAM4X_SHORT_CHUNK;
 constexpr unsigned char kNoSoa = 0xff;
 constexpr unsigned char kCapped = 0x80;  // bucket bit: the SOA loop hit its cap
 // bucket bit: the cell's loop left the range where the queue kernel's fast
@@ -144,31 +124,6 @@ __device__ __forceinline__ void ws_store_out(double *ws, long c, double g, const
   p[0] = Pair{g, a[0]};
   p[1] = Pair{a[1], a[2]};
   p[2] = Pair{a[3], gavg};
-}
-
-struct QueueCtl {
-  unsigned hist[kNBucket];  // cells per bucket
-  unsigned fill[kNBucket];  // scatter cursor per bucket
-  unsigned head;            // next free slot of the long part of the queue
-  unsigned pad[31];         // the two counters on separate cache lines
-  unsigned shead;           // next free slot of the short part
-};
-
-// The queue's granularity (mam4x_config.soa_chunk, soa_short_chunk,
-// soa_short_bucket; performance only): queue entries a wave takes per refill
-// from the long part and from the short part, the first bucket of the long
-// part, and the first bucket whose waves raise their issue priority.
-struct QueueShape {
-  int chunk, short_chunk, short_bucket, long_bucket;
-};
-
-static QueueShape queue_shape(const mam4x_config &c) {
-  QueueShape q;
-  q.chunk = c.soa_chunk > 0 ? c.soa_chunk : kChunk;
-  q.short_chunk = c.soa_short_chunk > 0 ? c.soa_short_chunk : kShortChunk;
-  q.short_bucket = c.soa_short_bucket > 0 ? c.soa_short_bucket : kShortBucket;
-  q.long_bucket = kLongBucket;
-  return q;
 }
 
 struct Work {
@@ -402,62 +357,9 @@ __global__ void __launch_bounds__(kBlock) queue_scatter_kernel(Work w) {
 // A wave exits once the queue is exhausted and all its lanes are idle; the
 // queue is finite and every cell ends after at most 1000 sub-steps, so every
 // wave exits.
-constexpr int kSeg = 32;      // records staged at a time
 constexpr int kRefill = 4;    // idle lanes that trigger a refill
 constexpr int kWaves = kBlock / 64;
 constexpr int kQuadLanes = 16;  // cells of a wave in QUAD form
-
-// The wave's source of queue entries: a claimed range, the next claim's
-// atomic in flight.  The long part of the queue first (the first claim of
-// every wave static: claim = wave index), then the short part.
-struct Claims {
-  unsigned beg, end;  // what is left of the claimed range (wave-uniform)
-  unsigned pend;      // lane 0: the outstanding atomic's result
-  bool longs, over;
-  unsigned nq, nsplit, chunk, short_chunk, first;
-  QueueCtl *ctl;
-  int lane;
-  __device__ __forceinline__ void ask() {
-    if (lane == 0) pend = atomicAdd(longs ? &ctl->head : &ctl->shead, longs ? chunk : short_chunk);
-  }
-  __device__ __forceinline__ void init(unsigned wid, unsigned nwave) {
-    first = nwave * chunk;
-    longs = true;
-    over = false;
-    pend = 0;
-    beg = min(wid * chunk, nsplit);
-    end = min(beg + chunk, nsplit);
-    if (first >= nsplit) longs = false;  // the static claims cover the long part
-    if (!longs && nsplit == nq)
-      over = beg == end;
-    else
-      ask();
-  }
-  // the next range of at most kSeg entries (empty: none left)
-  __device__ __forceinline__ void next(unsigned &b, unsigned &e) {
-    while (beg == end && !over) {
-      if (!longs && nsplit == nq) {
-        over = true;
-        break;
-      }
-      const unsigned v = __builtin_amdgcn_readfirstlane(pend) + (longs ? first : nsplit);
-      const unsigned lim = longs ? nsplit : nq;
-      if (v < lim) {
-        beg = v;
-        end = min(v + (longs ? chunk : short_chunk), lim);
-        ask();
-      } else if (longs) {
-        longs = false;
-        if (nsplit < nq) ask();
-      } else {
-        over = true;
-      }
-    }
-    b = beg;
-    e = min(beg + kSeg, end);
-    beg = e;
-  }
-};
 
 // Records on their way from the queue to the wave's LDS segment.  Lane l moves
 // the pairs (l & 7) of records l / 8, l / 8 + 8, ...; the place after a
@@ -2235,8 +2137,6 @@ static constexpr long kQuadCells = 163840;
 static void launch_soa_queue(mam4x_handle h, Work w, hipStream_t s) {
   w.quad = w.ncell <= kQuadCells;
   if (w.quad && !h->cfg.soa_chunk) w.qs.chunk = kQuadLanes;
-  // a wave's first claim starts at its index times the claim, in 32 bits
-  w.qs.chunk = std::min(w.qs.chunk, 1 << 18);
   const long claim = w.quad ? w.qs.chunk : std::min(w.qs.chunk, w.qs.short_chunk);
   const long waves = (w.ncell + claim - 1) / claim;
   const unsigned grid = (unsigned)std::min<long>(h->soa_grid, (waves + kWaves - 1) / kWaves);
