@@ -317,7 +317,11 @@ int mam4x_validate(mam4x_handle h, const mam4x_inputs *in, long long *violations
 
 /* AeroProcess<Impl>::compute_tendencies (aero_process.hpp:113-122) for all
  * columns: one chain step of length dt [s] followed by calcsize.  t is the
- * model time, unused (as in the reference). */
+ * model time, unused (as in the reference).  A graph that captured the step
+ * holds the handle's workspace: of up to 16,384 cells it stays valid until
+ * mam4x_destroy, of more until a call on the handle with a still larger domain
+ * (use mam4x_batch_create or the allocation-free step below to outlive that);
+ * its replays are calls on the handle, to be ordered with the others. */
 int mam4x_compute_tendencies(mam4x_handle h, double t, double dt,
                              const mam4x_inputs *in, const mam4x_outputs *out,
                              void *stream);

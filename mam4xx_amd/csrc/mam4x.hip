@@ -2069,15 +2069,12 @@ struct mam4x_handle_s {
   unsigned long long *d_count = nullptr;  // validate counter
   unsigned long long *d_stats = nullptr;  // SOA sub-steps since the last read
   bool stats = false;
-  // the buffers below d_consts to ctl, and a workspace for kFirstCells cells
+  // the buffers from d_consts to ctl, and the work-queue schedule's workspace
+  // for domains of up to kFirstCells cells
   unsigned char *base = nullptr, *first = nullptr;
-  // work-queue schedule: workspace for up to `cap` cells (grown on demand),
-  // `work` its own allocation, or NULL while it is `first` (in `base`)
+  // the workspace of larger domains, of up to `cap` cells (grown on demand)
   unsigned char *work = nullptr;
   long cap = 0;
-  double *ws = nullptr;
-  unsigned char *bucket = nullptr;
-  int *queue = nullptr;
   QueueCtl *ctl = nullptr;
   unsigned soa_grid = 0;  // resident blocks of soa_queue_kernel on the device
   int ncu = 0, soa_per_cu = 0;  // CUs, and the most SOA blocks one CU holds
@@ -2118,11 +2115,10 @@ static constexpr long kFirstCells = 16384;
 static constexpr size_t work_bytes(long ncell) {
   return (sizeof(double) * W_REC + sizeof(int) + 1) * (size_t)ncell;
 }
-static void set_work(mam4x_handle h, unsigned char *p, long ncell) {
-  h->ws = reinterpret_cast<double *>(p);
-  h->queue = reinterpret_cast<int *>(p + sizeof(double) * W_REC * ncell);
-  h->bucket = p + (sizeof(double) * W_REC + sizeof(int)) * ncell;
-  h->cap = ncell;
+static void set_work(Work &w, unsigned char *p, long ncell) {
+  w.ws = reinterpret_cast<double *>(p);
+  w.queue = reinterpret_cast<int *>(p + sizeof(double) * W_REC * ncell);
+  w.bucket = p + (sizeof(double) * W_REC + sizeof(int)) * ncell;
 }
 
 // Cells up to which soa_queue_kernel starts in its QUAD form.  Up to there the
@@ -2155,24 +2151,32 @@ static int fail(mam4x_handle h, int code, const std::string &msg) {
       return fail((h), MAM4X_ERR_HIP, std::string(#expr) + ": " + hipGetErrorString(e_)); \
   } while (0)
 
-// Workspace for ncell cells.  Growing frees an earlier allocation only after
-// the stream has drained, since earlier launches may still use it; the first
-// workspace stays with the handle.
-static int reserve_work(mam4x_handle h, long ncell, hipStream_t s) {
-  if (ncell <= h->cap) return MAM4X_OK;
-  if (h->work) {
-    HIP_TRY(h, hipStreamSynchronize(s));
-    (void)hipFree(h->work);
-    h->work = nullptr;
-    set_work(h, h->first, kFirstCells);
+// The workspace of a call on ncell cells: the first one, which stays where it
+// is as long as the handle lives (a captured step of a small domain holds its
+// address), or for a larger domain the growing one.  Growing frees the earlier
+// allocation only after the stream has drained, since earlier launches may
+// still use it.
+static int take_work(mam4x_handle h, long ncell, hipStream_t s, Work &w) {
+  if (ncell <= kFirstCells) {
+    set_work(w, h->first, kFirstCells);
+    return MAM4X_OK;
   }
-  if (hipMalloc(&h->work, work_bytes(ncell)) != hipSuccess) {
-    (void)hipGetLastError();
+  if (ncell > h->cap) {
+    if (h->work) {
+      HIP_TRY(h, hipStreamSynchronize(s));
+      (void)hipFree(h->work);
+    }
     h->work = nullptr;
-    return fail(h, MAM4X_ERR_NOMEM, "workspace allocation failed (" +
-                std::to_string(ncell) + " cells)");
+    h->cap = 0;
+    if (hipMalloc(&h->work, work_bytes(ncell)) != hipSuccess) {
+      (void)hipGetLastError();
+      h->work = nullptr;
+      return fail(h, MAM4X_ERR_NOMEM, "workspace allocation failed (" +
+                  std::to_string(ncell) + " cells)");
+    }
+    h->cap = ncell;
   }
-  set_work(h, h->work, ncell);
+  set_work(w, h->work, h->cap);
   return MAM4X_OK;
 }
 
@@ -2353,7 +2357,6 @@ int mam4x_create(const mam4x_config *config, mam4x_handle *out) {
   h->d_stats = reinterpret_cast<unsigned long long *>(p += kAlign);
   h->ctl = reinterpret_cast<QueueCtl *>(p += kAlign);
   h->first = p + kCtlBytes;
-  set_work(h, h->first, kFirstCells);
   if (hipMemcpy(h->d_consts, &k, sizeof(k), hipMemcpyHostToDevice) != hipSuccess ||
       hipMemset(h->d_stats, 0, sizeof(unsigned long long)) != hipSuccess) {
     mam4x_destroy(h);
@@ -2577,11 +2580,8 @@ int mam4x_compute_tangent(mam4x_handle h, double t, double dt, const mam4x_input
   if (a.cfg.do_cond) {
     // cells in the work queue's order (the FP64 set-up kernel predicts each
     // cell's SOA cost): a wave's lanes then run loops of similar length
-    rc = reserve_work(h, ncell, s);
+    rc = take_work(h, ncell, s, w);
     if (rc) return rc;
-    w.ws = h->ws;
-    w.bucket = h->bucket;
-    w.queue = h->queue;
     w.ctl = h->ctl;
     w.dtfull = dev::dt_sub(a.cfg, dt);
     hipLaunchKernelGGL(queue_reset_kernel, dim3(1), dim3(64), 0, s, w.ctl);
@@ -2688,23 +2688,20 @@ int mam4x_compute_adjoint(mam4x_handle h, double t, double dt, const mam4x_input
     const QueueCtl *ctl = nullptr;
     if (a.cfg.do_cond) {
       // the first sub-step's predicted SOA cost orders the cells
-      rc = reserve_work(h, ncell, s);
-      if (rc) return rc;
       Work w;
       std::memset(&w, 0, sizeof(w));
+      rc = take_work(h, ncell, s, w);
+      if (rc) return rc;
       w.qs = queue_shape(h->cfg);
       w.ncell = ncell;
       w.ctl = h->ctl;
       w.dtfull = dev::dt_sub(a.cfg, dt);
-      w.ws = h->ws;
-      w.bucket = h->bucket;
-      w.queue = h->queue;
       hipLaunchKernelGGL(queue_reset_kernel, dim3(1), dim3(64), 0, s, h->ctl);
       launch_cells<Fp64>(kPre, pre, grid, s, OneDomain{a}, w);
       hipLaunchKernelGGL(queue_scatter_kernel, dim3(scatter_grid(w.ncell)), dim3(kBlock), 0, s, w);
-      queue = h->queue;
+      queue = w.queue;
       ctl = h->ctl;
-      o.bucket = h->bucket;
+      o.bucket = w.bucket;
       if (pre)
         hipLaunchKernelGGL((chain_adjoint_sub_kernel<true>), dim3(grid), dim3(kBlock), 0, s, a,
                            o, h->subws, queue, ctl, 0);
@@ -2722,7 +2719,9 @@ int mam4x_compute_adjoint(mam4x_handle h, double t, double dt, const mam4x_input
     return MAM4X_OK;
   }
   if (a.cfg.do_cond) {
-    rc = reserve_work(h, ncell, s);
+    Work w;
+    std::memset(&w, 0, sizeof(w));
+    rc = take_work(h, ncell, s, w);
     if (rc) return rc;
     rc = reserve_adjoint(h, ncell, s);
     if (rc) return rc;
@@ -2737,15 +2736,10 @@ int mam4x_compute_adjoint(mam4x_handle h, double t, double dt, const mam4x_input
       if (rc) return rc;
     }
     // 1. set-up and queue
-    Work w;
-    std::memset(&w, 0, sizeof(w));
     w.qs = queue_shape(h->cfg);
     w.ncell = ncell;
     w.ctl = h->ctl;
     w.dtfull = (double)(int)(dt / 1);  // QUIRK (mam4_amicphys.hpp:1319): int sub-step
-    w.ws = h->ws;
-    w.bucket = h->bucket;
-    w.queue = h->queue;
     const OneDomain src{a};
     hipLaunchKernelGGL(queue_reset_kernel, dim3(1), dim3(64), 0, s, h->ctl);
     launch_cells<Fp64>(kPre, pre, grid, s, src, w);
@@ -2753,15 +2747,15 @@ int mam4x_compute_adjoint(mam4x_handle h, double t, double dt, const mam4x_input
     HIP_TRY(h, hipGetLastError());
     AdjWork g;
     g.qs = queue_shape(h->cfg);
-    g.ws = h->ws;
+    g.ws = w.ws;
     g.res = h->adjws;
     g.pb = h->adjws + (size_t)R_NPLANE * ncell;
     g.inb = h->adjws + (size_t)(R_NPLANE + kPbPlanes) * ncell;
     g.wend = h->log_wend;
     g.next = h->log_next;
     g.nwave = h->log_grid * (kBlock / 64);
-    g.bucket = h->bucket;
-    g.queue = h->queue;
+    g.bucket = w.bucket;
+    g.queue = w.queue;
     g.ctl = h->ctl;
     g.ncell = ncell;
     g.dtfull = w.dtfull;
@@ -2794,7 +2788,7 @@ int mam4x_compute_adjoint(mam4x_handle h, double t, double dt, const mam4x_input
       hipLaunchKernelGGL((adj_pre_kernel<true>), dim3(grid), dim3(kBlock), 0, s, a, g, o);
     else
       hipLaunchKernelGGL((adj_pre_kernel<false>), dim3(grid), dim3(kBlock), 0, s, a, g, o);
-    o.bucket = h->bucket;  // the rest: overcast cells
+    o.bucket = w.bucket;  // the rest: overcast cells
   }
   if (pre)
     hipLaunchKernelGGL((chain_adjoint_kernel<true>), dim3(grid), dim3(kBlock), 0, s, a, o);
@@ -3030,11 +3024,8 @@ static int compute_step(mam4x_handle h, double dt, const mam4x_inputs *in,
     w.queue = reinterpret_cast<int *>(h->scratch + kScratchQueueOff);
     w.bucket = h->scratch + kScratchBucketOff;
   } else if (queue) {
-    rc = reserve_work(h, ncell, s);
+    rc = take_work(h, ncell, s, w);
     if (rc) return rc;
-    w.ws = h->ws;
-    w.bucket = h->bucket;
-    w.queue = h->queue;
   }
   hipEvent_t *ev = nullptr;
   if (h->stats && !noalloc) {
