@@ -2029,7 +2029,9 @@ static void launch_order(bool pre, unsigned grid, hipStream_t s, const OneDomain
 // the work-queue workspace for up to kScratchCells cells -- W_REC doubles
 // a cell, the queue, the cost buckets -- and the queue counters.  Every GPU the
 // library runs on holds one copy (117 B per cell: 61.3 MB) until the process
-// ends; every call on a GPU shares it, so calls that overlap on one GPU race.
+// ends; every call of more than kFirstCells cells on a GPU shares it, so such
+// calls that overlap on one GPU race.  Smaller domains use their handle's own
+// first workspace.
 static constexpr long kScratchCells = MAM4X_NOALLOC_MAX_CELLS;
 static constexpr size_t kScratchWsBytes = sizeof(double) * W_REC * kScratchCells;
 static constexpr size_t kScratchQueueOff = kScratchWsBytes;
@@ -2968,8 +2970,9 @@ static int launch_budgets(mam4x_handle h, const mam4x_inputs *in, const mam4x_ou
 }
 
 // One step on one domain.  With noalloc the work-queue workspace and its
-// counters live in the device's `scratch` array and no phase events are
-// recorded: the call allocates nothing and only launches kernels.
+// counters live in the device's `scratch` array (small domains: in the handle)
+// and no phase events are recorded: the call allocates nothing and only launches
+// kernels.
 static int compute_step(mam4x_handle h, double dt, const mam4x_inputs *in,
                         const mam4x_outputs *out, void *stream, bool noalloc) {
   int rc = check_inputs(h, in);
@@ -3013,12 +3016,13 @@ static int compute_step(mam4x_handle h, double dt, const mam4x_inputs *in,
   std::memset(&w, 0, sizeof(w));
   w.qs = queue_shape(h->cfg);
   w.ncell = ncell;
-  w.ctl = noalloc ? reinterpret_cast<QueueCtl *>(h->scratch + kScratchCtlOff) : h->ctl;
+  const bool shared = noalloc && ncell > kFirstCells;  // take_work would allocate
+  w.ctl = shared ? reinterpret_cast<QueueCtl *>(h->scratch + kScratchCtlOff) : h->ctl;
   w.dtfull = dev::dt_sub(a.cfg, dt);  // QUIRK (mam4_amicphys.hpp:1319): int sub-step
   if (h->stats) w.stats = h->d_stats;
   const OneDomain src{a};
   const bool queue = !fused && a.cfg.do_cond;
-  if (queue && noalloc) {
+  if (queue && shared) {
     // ncell records fit the kScratchCells-sized region
     w.ws = reinterpret_cast<double *>(h->scratch);
     w.queue = reinterpret_cast<int *>(h->scratch + kScratchQueueOff);

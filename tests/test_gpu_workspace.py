@@ -1,6 +1,7 @@
 """A handle's workspace: a captured step of a small domain holds the address of
 the handle's first workspace, which stays where it is while larger domains make
-the handle's other workspace grow and move."""
+the handle's other workspace grow and move; and the allocation-free steps of
+small domains on two handles share nothing."""
 import pytest
 
 from mam4xx_amd import layout as L
@@ -47,6 +48,31 @@ def test_captured_small_step_survives_growth(torch_cuda, ncol, nlev):
             assert torch.equal(out, want)
     del graph
     ch.close()
+    ref.close()
+
+
+def test_noalloc_small_steps_of_two_handles_overlap(torch_cuda):
+    """each handle on a stream of its own, nothing ordering the two"""
+    from mam4xx_amd.chain import Chain
+    torch = torch_cuda
+    ref = Chain()
+    jobs = []
+    for i, ncol in enumerate((96, 200)):
+        d, want = _scene(torch, ncol, 72, 40 + i)
+        ref.compute_tendencies(d, DT, want)
+        torch.cuda.synchronize()
+        jobs.append((Chain(), torch.cuda.Stream(), d, want,
+                     [torch.full_like(want, float("nan")) for _ in range(8)]))
+    torch.cuda.synchronize()
+    for k in range(8):
+        for ch, stream, d, _, outs in jobs:
+            with torch.cuda.stream(stream):
+                ch.compute_tendencies(d, DT, outs[k], noalloc=True)
+    torch.cuda.synchronize()
+    for ch, _, _, want, outs in jobs:
+        for out in outs:
+            assert torch.equal(out, want)
+        ch.close()
     ref.close()
 
 
