@@ -17,25 +17,58 @@ vapour.
 Derivatives are those of the branch each cell takes (include/mam4x.h,
 mam4x_compute_tangent).
 """
+import contextlib
+import threading
+
 import torch
 
+from . import _abi
 from . import layout as L
 from .chain import Chain
 
-# One handle per device and stream: calls on a handle share its workspace, so
-# they have to be ordered.  The oldest goes when there are _MOST_CHAINS (its
-# memory is freed once the device has finished with it).
-_MOST_CHAINS = 64
-_chains = {}
+# A captured forward step of fewer cells runs the fused kernel, which has no
+# workspace: its replays need no ordering with the other calls, on any stream.
+# Eagerly the work queue is faster (include/mam4x.h, MAM4X_SCHED_AUTO).
+_CAPTURED_FUSED = 16384
 
 
-def _chain():
-    key = torch.cuda.current_device(), torch.cuda.current_stream().cuda_stream
-    if key not in _chains:
-        if len(_chains) >= _MOST_CHAINS:
-            del _chains[next(iter(_chains))]
-        _chains[key] = Chain()
-    return _chains[key]
+class _Handles:
+    """A device's handles, made outside captures (a capture allows no
+    allocation) and kept: `chain` for every call, `fused` for captured small
+    steps.  Calls on a handle share its workspace, so each waits for the one
+    before, whatever their streams and threads."""
+
+    def __init__(self):
+        self.chain, self.fused = Chain(), Chain(schedule=_abi.SCHED_FUSED)
+        self.last = torch.cuda.Event()
+        self.lock = threading.Lock()
+
+
+_handles = {}
+_handles_lock = threading.Lock()
+
+
+@contextlib.contextmanager
+def _handle(ncell=None):
+    """The current device's handle, for launches on the current stream; ncell:
+    the cells of a forward step.  Captured calls only have the graph's order:
+    replays that use the workspace (derivatives, larger steps) have to be
+    ordered with other calls by the caller."""
+    dev = torch.cuda.current_device()
+    with _handles_lock:
+        if dev not in _handles:
+            _handles[dev] = _Handles()
+        h = _handles[dev]
+    with h.lock:
+        if torch.cuda.is_current_stream_capturing():
+            yield h.fused if ncell is not None and ncell < _CAPTURED_FUSED else h.chain
+            return
+        stream = torch.cuda.current_stream()
+        stream.wait_event(h.last)
+        try:
+            yield h.chain
+        finally:
+            h.last.record(stream)
 
 
 def _scene(scene, state, temperature, pressure, qv):
@@ -51,8 +84,9 @@ def _tangent(d, dt, dstate, dT, dp, dqv):
     nlev, ncol = d["temperature"].shape
     tend = torch.empty((L.NSTATE, nlev, ncol), dtype=torch.float64, device="cuda")
     dtend = torch.empty_like(tend)
-    _chain().compute_tangent(d, dt, tend, dtend, dstate=dstate, dtemperature=dT, dpressure=dp,
-                             dqv=dqv)
+    with _handle() as ch:
+        ch.compute_tangent(d, dt, tend, dtend, dstate=dstate, dtemperature=dT, dpressure=dp,
+                           dqv=dqv)
     return tend, dtend
 
 
@@ -62,7 +96,8 @@ class _Tendencies(torch.autograd.Function):
         d = _scene(scene, state, temperature, pressure, qv)
         nlev, ncol = d["temperature"].shape
         tend = torch.empty((L.NSTATE, nlev, ncol), dtype=torch.float64, device="cuda")
-        _chain().compute_tendencies(d, dt, tend)
+        with _handle(nlev * ncol) as ch:
+            ch.compute_tendencies(d, dt, tend)
         return tend
 
     @staticmethod
@@ -91,8 +126,9 @@ class _Tendencies(torch.autograd.Function):
         for k in (1, 2, 3):
             if ctx.needs_input_grad[k]:
                 grads[k] = new(nlev, ncol)
-        _chain().compute_adjoint(d, dt, g, state_bar=grads[0], temperature_bar=grads[1],
-                                 pressure_bar=grads[2], qv_bar=grads[3])
+        with _handle() as ch:
+            ch.compute_adjoint(d, dt, g, state_bar=grads[0], temperature_bar=grads[1],
+                               pressure_bar=grads[2], qv_bar=grads[3])
         return grads[0], grads[1], grads[2], grads[3], None, None
 
 
