@@ -1902,13 +1902,14 @@ __global__ void __launch_bounds__(kPhotoColBlock) photo_column_kernel(PhotoArgs 
 // angle, ozone ratio, albedo and pressure, in pairs along the albedo, and two
 // of the cross section around its temperature and pressure.  Neighbouring
 // columns differ in all of these but pressure, so a gather touches up to 64
-// lines and the lines' traffic bounds the pass.  A block therefore first puts
-// its cells in order of their zenith angle's and ozone ratio's places: the
-// lanes of a wave then read the same few lines, and the dark columns' lanes
-// come last, in waves that end at once.  21,600 x 72, a fifth of the columns
-// dark: 0.82 ms as the cells come, 0.72 with pairs, 0.52 with the order (0.62
-// in blocks of 1024).  Staging a wavelength's pressure layers in LDS took 0.68
-// ms without the order and 0.55 with it, bound by the banks.
+// lines and the lines' traffic bounds the pass.  photo_level_order_kernel
+// therefore first puts a block's cells in order of their zenith angle's and
+// ozone ratio's places: the lanes of a wave then read the same few lines, and
+// the dark columns' lanes come last, in waves that end at once.  21,600 x 72, a
+// fifth of the columns dark: 0.82 ms as the cells come, 0.52 with the order
+// (0.62 in blocks of 1024); level-fastest 4.08 ms and 0.87.  Staging a
+// wavelength's pressure layers in LDS took 0.68 ms without the order and 0.55
+// with it, bound by the banks.
 constexpr int kPhotoBlock = 512;
 constexpr int kPhotoKeys = 128;  // groups of a block's cells; the last: dark or no cell
 constexpr int kPhotoLev = 4;     // COL_LEV: a block is 4 levels x 128 columns
@@ -1921,7 +1922,49 @@ static unsigned photo_level_grid(int ncol, int nlev, int layout) {
   return (unsigned)(((long)ncol * nlev + kPhotoBlock - 1) / kPhotoBlock);
 }
 
-__global__ void __launch_bounds__(kPhotoBlock) photo_level_kernel(PhotoArgs a) {
+// The same with a cell to each lane as they come.
+__global__ void __launch_bounds__(kBlock) photo_level_kernel(PhotoArgs a) {
+  const long c = (long)blockIdx.x * kBlock + threadIdx.x;
+  if (c >= (long)a.ncol * a.nlev) return;
+  const bool cl = a.layout == MAM4X_LAYOUT_COL_LEV;
+  const int fast = cl ? a.nlev : a.ncol;
+  const long slow = c / fast;
+  const int f = (int)(c - slow * fast);
+  const int j = cl ? (int)slow : f;
+  const long off = slow * a.ldc + f;
+  const double sza = pht::sza_deg(a.zen[j]);
+  if (!pht::daylight(sza)) return;
+  const double jr = pht::level_rate(a.t, pht::sza_pos(a.t, sza), a.eff[off],
+                                    a.pmid[off] * pht::kPaToMb, a.T[off], a.colo3[off]);
+  a.photo[off] = pht::update(a.t, a.photo[off], a.mult[off], a.esfact, jr);
+}
+
+// Whether the order pays: its passes take some 10 us, and larger blocks fill the
+// chip later.  us as the cells come / in order, with wavelengths x pressures x
+// zenith angles x ozone ratios x albedos:
+//   column-fastest, 67 x 51 x 10 x 10 x 6 (16 MB): 16 x 72 80 / 197, 400 x 72
+//     84 / 91, 1,000 x 72 121 / 96, 5,400 x 72 247 / 170; 120 wavelengths (29 MB)
+//     1.2 to 1.6 times faster from 1,000 x 72; 20 (5 MB) 66 / 70 at 2,700 x 72,
+//     99 / 86 at 5,400; 8: 170 / 207 at 21,600; a table of 67 x 5 x 3 x 4 x 3
+//     137 / 140 at 4,000 x 72, 160 / 142 at 5,400;
+//   with more places than groups (20 x 20) 606 / 705 at 4,000 x 72, 2,357 /
+//     2,455 at 21,600 (13 x 10: 166 / 139 at 2,700);
+//   level-fastest, 16 MB: 156 / 79 at 16 x 72, 145 / 102 at 400, 450 / 174 at
+//     2,700; 5 MB 69 / 65 at 400, 99 / 66 at 1,000; 8 wavelengths 79 / 75 at
+//     4,000; the smallest table 228 / 275 at 2,700, 438 / 365 at 4,000; 20 x 20
+//     places 238 / 270 at 400, 480 / 277 at 1,000; three levels 63 / 72, sixteen
+//     83 / 88, twenty-six 153 / 106.
+static bool photo_ordered(const PhotoArgs &a) {
+  const long ncell = (long)a.ncol * a.nlev;
+  const double mb = 8e-6 * a.t.nw * a.t.nump * a.t.numsza * a.t.numcolo3 * a.t.numalb;
+  const bool places = (long)a.t.numsza * a.t.numcolo3 <= kPhotoKeys + kPhotoKeys / 4;
+  if (a.layout == MAM4X_LAYOUT_COL_LEV)
+    return a.nlev >= 24 &&
+           ncell >= (mb >= 8.0 && places ? 1024 : mb >= 4.0 ? 65536 : 262144);
+  return places && a.t.nw >= 20 && ncell >= (mb >= 12.0 ? 65536 : 327680);
+}
+
+__global__ void __launch_bounds__(kPhotoBlock) photo_level_order_kernel(PhotoArgs a) {
   __shared__ int cnt[kPhotoKeys], base[kPhotoKeys], order[kPhotoBlock];
   const int tid = threadIdx.x;
   int j = 0;
@@ -3441,9 +3484,13 @@ int mam4x_compute_photolysis(mam4x_handle h, const mam4x_photo_table *tb,
     hipLaunchKernelGGL(photo_column_kernel,
                        dim3((unsigned)((in->ncol + kPhotoColBlock - 1) / kPhotoColBlock)),
                        dim3(kPhotoColBlock), 0, (hipStream_t)stream, a);
-  hipLaunchKernelGGL(photo_level_kernel,
-                     dim3(photo_level_grid(in->ncol, in->nlev, in->layout)), dim3(kPhotoBlock), 0,
-                     (hipStream_t)stream, a);
+  if (photo_ordered(a))
+    hipLaunchKernelGGL(photo_level_order_kernel,
+                       dim3(photo_level_grid(in->ncol, in->nlev, in->layout)), dim3(kPhotoBlock),
+                       0, (hipStream_t)stream, a);
+  else
+    hipLaunchKernelGGL(photo_level_kernel, dim3((unsigned)((ncell + kBlock - 1) / kBlock)),
+                       dim3(kBlock), 0, (hipStream_t)stream, a);
   HIP_TRY(h, hipGetLastError());
   return MAM4X_OK;
 }

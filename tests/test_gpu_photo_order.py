@@ -1,8 +1,8 @@
-"""The photolysis level pass puts a block's cells in an order of its own, which
-must not show: a domain, its columns taken a few at a time and the level-fastest
-layout (blocked by tiles of levels and columns) give the same bits, with domains
-off the block's sizes, dark columns, one cell, and tables with more places than
-the order has groups."""
+"""Where it pays, the photolysis level pass puts a block's cells in an order of its
+own, which must not show: a domain, its columns taken a few at a time (as they
+come) and the level-fastest layout (blocked by tiles of levels and columns) give
+the same bits, with domains off the block's sizes, dark columns, one cell, and
+tables with more places than the order has groups."""
 import numpy as np
 import pytest
 
@@ -32,9 +32,14 @@ def rates(torch, t, cols, sel, col_lev):
     return r.T if col_lev else r
 
 
-@pytest.mark.parametrize("ncol,nlev,axes", [(1537, 72, "wide"), (513, 5, "wide"), (700, 31, "ref"),
-                                            (1, 1, "wide"), (129, 73, "fine")])
-def test_the_blocks_order_does_not_show(ncol, nlev, axes):
+# the last five in order: either layout (16 MB, 120 x 547 cells), level-fastest
+# (10 MB from 1,024 cells; 400 places from 65,536; a small table from 262,144)
+@pytest.mark.parametrize("ncol,nlev,axes,nw", [
+    (1537, 72, "wide", 5), (513, 5, "wide", 5), (700, 31, "ref", 5), (1, 1, "wide", 5),
+    (129, 73, "fine", 5),
+    (547, 120, "wide", 67), (129, 73, "wide", 40), (43, 24, "wide", 40), (911, 72, "fine", 4),
+    (3651, 72, "ref", 5)])
+def test_the_blocks_order_does_not_show(ncol, nlev, axes, nw):
     import torch
     if not torch.cuda.is_available():
         pytest.fail("GPU test run without a GPU")
@@ -42,7 +47,7 @@ def test_the_blocks_order_does_not_show(ncol, nlev, axes):
     ax = dict(wide=PT.wide_axes(), ref=PT.REF_AXES,
               # more places than groups
               fine=PT.wide_axes(numsza=20, numcolo3=20, numalb=12))[axes]
-    t = PT.random_table(rng, ax, nw=5)
+    t = PT.random_table(rng, ax, nw=nw)
     cols = PT.columns(rng, nlev, ncol, PT.wide_axes())
     cols["temp"][:, :: 7] = rng.uniform(120.0, 380.0, cols["temp"][:, :: 7].shape)
     a = rates(torch, t, cols, np.arange(ncol), False)
