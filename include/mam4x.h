@@ -97,7 +97,8 @@ extern "C" {
 #define MAM4X_LAYOUT_COL_LEV 1
 
 /* schedule of a step (performance only; results are identical) */
-#define MAM4X_SCHED_AUTO 0  /* the faster for the domain: the work queue    */
+#define MAM4X_SCHED_AUTO 0  /* the work queue; below 16,384 cells fused for  */
+                            /* steps under 60 s or with ntsubstep > 1       */
 #define MAM4X_SCHED_FUSED 1 /* one lane runs one cell's whole step         */
 #define MAM4X_SCHED_QUEUE 2 /* per-cell phases around a work-queue kernel  */
                             /* that runs the SOA sub-stepping              */

@@ -20,7 +20,8 @@
 //                         next cell as soon as its current one has converged
 //   4. chain_post_kernel  per cell: the rest of the chain, recombination,
 //                         calcsize, tendencies
-// chain_fused_kernel runs everything in one lane per cell (MAM4X_SCHED_FUSED).
+// chain_fused_kernel runs everything in one lane per cell (MAM4X_SCHED_FUSED, and
+// short steps of small domains).
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -2144,8 +2145,19 @@ struct mam4x_handle_s {
   std::string err;
 };
 
-// cells below which MAM4X_SCHED_AUTO takes the fused kernel for ntsubstep > 1
+// MAM4X_SCHED_AUTO takes the fused kernel for domains of fewer than kFusedBelow
+// cells with ntsubstep > 1 (one lane runs a cell either way) or steps so short
+// that no SOA chain is long.  Otherwise the queue, also for the smallest: its
+// QUAD form halves the longest chain.  us a step, fused / queue, at 72 levels:
+// 1 column dt = 1 s 54 / 67, 30 s 64 / 74, 60 s 74 / 77, 1800 s 280 / 177; 16
+// columns 56 / 71, 97 / 97, 147 / 123, 444 / 306; 200 columns 57 / 73, 98 / 104,
+// 153 / 133, 922 / 476.
 static constexpr long kFusedBelow = 16384;
+static constexpr double kFusedDt = 60.0;  // the loop's length [s]
+static bool auto_fused(const mam4x_config &c, long ncell, bool multi, double dtfull) {
+  return c.schedule == MAM4X_SCHED_FUSED ||
+         (c.schedule == MAM4X_SCHED_AUTO && ncell < kFusedBelow && (multi || dtfull < kFusedDt));
+}
 
 static void destroy_events(mam4x_handle h) {
   for (auto *v : {&h->pending, &h->pool})
@@ -2170,13 +2182,17 @@ static void set_work(Work &w, unsigned char *p, long ncell) {
 // longest chains set its time and the chip has issue slots to spare; beyond,
 // the work does.  One-lane against QUAD form, ms per step at 72 levels: 1000
 // columns 0.736 / 0.653, 2000 0.823 / 0.797, 2701 0.842 / 0.868, 5400 1.150 /
-// 1.426.
-static constexpr long kQuadCells = 163840;
+// 1.426.  Short steps have no long chains, so their work sets the time of
+// smaller launches already (us): 1000 columns dt = 1 s 133 / 157, 5 s 156 / 159,
+// 20 s 218 / 179; 2000 columns 206 / 268, 10 s 259 / 270, 20 s 297 / 278; 400
+// columns 98 / 80.
+static constexpr long kQuadCells = 163840, kQuadCellsShort = 65536;
+static constexpr double kQuadDt = 20.0;  // the loop's length [s]
 
 // soa_queue_kernel over w.ncell cells: its form, its claims (16 cells fill a
 // wave in QUAD form) and its grid, no larger than its claims need
 static void launch_soa_queue(mam4x_handle h, Work w, hipStream_t s) {
-  w.quad = w.ncell <= kQuadCells;
+  w.quad = w.ncell <= (w.dtfull < kQuadDt ? kQuadCellsShort : kQuadCells);
   if (w.quad && !h->cfg.soa_chunk) w.qs.chunk = kQuadLanes;
   const long claim = w.quad ? w.qs.chunk : std::min(w.qs.chunk, w.qs.short_chunk);
   const long waves = (w.ncell + claim - 1) / claim;
@@ -3045,23 +3061,18 @@ static int compute_step(mam4x_handle h, double dt, const mam4x_inputs *in,
   const long ncell = (long)in->ncol * in->nlev;
   if (ncell == 0) return out->column_budgets ? launch_budgets(h, in, out, s) : MAM4X_OK;
   const unsigned grid = (unsigned)((ncell + kBlock - 1) / kBlock);
-  // the queue also for the smallest domains: its QUAD form halves the longest
-  // SOA chain (1 column x 72: 0.262 ms a step against 0.452 fused, 16: 0.551 /
-  // 0.867, 200: 0.573 / 1.372)
-  // (one sub-step; with more, one lane runs a cell either way)
-  const bool fused =
-      h->cfg.schedule == MAM4X_SCHED_FUSED ||
-      (h->cfg.schedule == MAM4X_SCHED_AUTO && dev::nsub(a.cfg) > 1 && ncell < kFusedBelow);
   // ntsubstep > 1: one lane runs a cell's whole step (the split phases hold
   // one sub-step), in the queue's order unless the fused schedule is chosen
   const bool multi = dev::nsub(a.cfg) > 1;
+  const double dtfull = dev::dt_sub(a.cfg, dt);  // QUIRK (mam4_amicphys.hpp:1319): int sub-step
+  const bool fused = auto_fused(h->cfg, ncell, multi, dtfull);
   Work w;
   std::memset(&w, 0, sizeof(w));
   w.qs = queue_shape(h->cfg);
   w.ncell = ncell;
   const bool shared = noalloc && ncell > kFirstCells;  // take_work would allocate
   w.ctl = shared ? reinterpret_cast<QueueCtl *>(h->scratch + kScratchCtlOff) : h->ctl;
-  w.dtfull = dev::dt_sub(a.cfg, dt);  // QUIRK (mam4_amicphys.hpp:1319): int sub-step
+  w.dtfull = dtfull;
   if (h->stats) w.stats = h->d_stats;
   const OneDomain src{a};
   const bool queue = !fused && a.cfg.do_cond;
@@ -3622,8 +3633,8 @@ int mam4x_batch_create(mam4x_handle h, int nscene, const mam4x_inputs *in,
       b->budgets.emplace_back();
       budget_args(&in[i], &out[i], b->budgets.back());
     }
-  b->fused = h->cfg.schedule == MAM4X_SCHED_FUSED ||
-             h->cfg.ntsubstep > 1;  // the split phases hold one sub-step
+  b->fused = h->cfg.ntsubstep > 1 ||  // the split phases hold one sub-step
+             auto_fused(h->cfg, b->ncell, false, (double)(int)(dt / 1));
   b->queue = !b->fused && args[0].cfg.do_cond != 0 && b->ncell > 0;
   if (hipMalloc(&b->d_args, sizeof(ChainArgs) * nscene) != hipSuccess ||
       hipMalloc(&b->d_blk0, sizeof(unsigned) * (nscene + 1)) != hipSuccess ||

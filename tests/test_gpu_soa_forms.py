@@ -48,3 +48,30 @@ def test_queue_forms_equal_the_fused_kernel(ncol, nlev, cfg):
     for t, cap in out[1:]:
         assert np.array_equal(t.view(np.int64), out[0][0].view(np.int64))
         assert np.array_equal(cap, out[0][1])
+
+
+@pytest.mark.parametrize("ncol,dt", [(3, 59.9), (3, 60.0), (227, 1.0), (227, 30.0), (228, 30.0),
+                                     (911, 19.9), (911, 20.0), (1000, 0.5)])
+def test_short_steps_take_the_same_values(ncol, dt):
+    """either side of the rules on the step's length (72 levels: 227 columns are
+    the last of fewer than 16,384 cells, 911 the first of more than 65,536)"""
+    import torch
+    from mam4xx_amd import _abi
+    from mam4xx_amd.chain import Chain, scene_to_device
+    if not torch.cuda.is_available():
+        pytest.fail("GPU test run without a GPU")
+    d = scene_to_device(scenes.generate(ncol, 72, seed=9))
+    out = []
+    for kw in (dict(schedule=_abi.SCHED_FUSED), dict(schedule=_abi.SCHED_QUEUE), {}):
+        ch = Chain(**kw)
+        t = [torch.full((L.NSTATE, 72, ncol), float("nan"), dtype=torch.float64, device="cuda")
+             for _ in range(2)]
+        ch.compute_tendencies(d, dt, t[0])
+        b = ch.batch([d], dt, [t[1]])
+        b.run()
+        torch.cuda.synchronize()
+        out += [x.cpu().numpy().view(np.int64) for x in t]
+        b.close()
+        ch.close()
+    for t in out[1:]:
+        assert np.array_equal(t, out[0])
