@@ -376,14 +376,14 @@ __device__ __forceinline__ int soa_state_exp(const SoaState<double> &s) {
 __device__ __forceinline__ int soa_state_exp(const SoaState<num::Dual> &) { return 0; }
 
 // ---- the FAST sub-step on bounded inputs
-// SoaRun is the loop of one cell whose inputs passed soa_run_ok: every mass is
-// 0 or in [2^-400, 2^8] to begin with, a skipped mode (uptake <= 1e-15) has
-// uk = a = 0, the loop runs at least one sub-step, and the two modes whose
-// oxygenated POM soa_in_state makes 0 have none.  The masses then stay
-// >= 0 and finite, so soa_run_tick leaves out the clips of a state at 0, the
-// skip selects and the leading 0 + x of the sums, and takes vmax for kmax (the
-// larger of three in any order): every value equals soa_tick<true>'s bit for
-// bit.
+// SoaRun is the loop of one cell whose inputs soa_run_cell and soa_run_mode
+// accepted: every mass is 0 or in [2^-400, 2^8] to begin with, a skipped mode
+// (uptake <= 1e-15) has uk = a = 0, the loop runs at least one sub-step, and the
+// two modes whose oxygenated POM soa_in_state makes 0 have none.  The masses
+// then stay >= 0 and finite, so soa_run_tick leaves out the clips of a state at
+// 0, the skip selects and the leading 0 + x of the sums, and takes vmax for kmax
+// (the larger of three in any order): every value equals soa_tick<true>'s bit
+// for bit.
 //
 // low is the smallest high word minus one (unsigned, so that a zero counts as
 // large) among the states' masses: the record soa_fast_exact needs.  A state

@@ -50,16 +50,6 @@ using namespace mam4x;
 namespace {
 
 constexpr int kBlock = 256;
-// Waves whose first chunk comes from buckets >= kLongBucket (predicted >= ~180
-// sub-steps) raise their issue priority: a cell's sub-steps are a serial
-// chain, so the longest cells set the kernel's critical path and should not
-// yield issue slots to the bulk.
-#ifndef MAM4X_SOA_PRIO
-#define MAM4X_SOA_PRIO 1
-#endif
-#ifndef MAM4X_STATIC_FIRST
-#define MAM4X_STATIC_FIRST 1
-#endif
 // Minimum waves per SIMD the reverse sweep's heaviest kernels are compiled
 // for (1: as many registers as the compiler wants).
 #ifndef MAM4X_REPLAY_WAVES
@@ -732,8 +722,9 @@ __device__ __forceinline__ void pb_store(double *pl, long n, long c,
   for (int m = 0; m < 4; ++m) q[(long)(kPbSoa + 2 + m) * n] = pb.soa_a_b[m];
 }
 
-// Phase 2: soa_queue_kernel's loop (same refill, same sub-steps) with the
-// log written at the end of every iteration.  A pool that runs out stops the
+// Phase 2: the SOA loop over the work queue, a lane to a cell and each lane
+// fetching its own record (soa_queue_kernel's values, without its staging), with
+// the log written at the end of every iteration.  A pool that runs out stops the
 // wave's logging, but the loop still drains the queue and still counts the
 // chunks it would have taken: the caller sees *next > cap, the pool this
 // run needed, and runs the phase again with a pool that large.
@@ -747,7 +738,7 @@ __global__ void __launch_bounds__(kBlock) soa_log_kernel(AdjWork g) {
   const unsigned qchunk = (unsigned)g.qs.chunk, qschunk = (unsigned)g.qs.short_chunk;
   const unsigned nwave = gridDim.x * (kBlock / 64);
   const unsigned wid = blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6);
-  bool first = MAM4X_STATIC_FIRST != 0;
+  bool first = true;
   const int lane = threadIdx.x & 63;
   const long n = g.ncell;
   unsigned cbeg = 0, cend = 0;  // the wave's current chunk of the queue (wave-uniform)
@@ -766,8 +757,7 @@ __global__ void __launch_bounds__(kBlock) soa_log_kernel(AdjWork g) {
         b0 = wid * qchunk;
       } else if (!lexhausted) {
         if (lane == 0) b0 = atomicAdd(&g.ctl->head, qchunk);
-        b0 = (MAM4X_STATIC_FIRST ? nwave * qchunk : 0u) +
-             __builtin_amdgcn_readfirstlane(b0);
+        b0 = nwave * qchunk + __builtin_amdgcn_readfirstlane(b0);
       }
       if (b0 < nsplit) {
         e0 = min(b0 + qchunk, nsplit);
@@ -777,7 +767,7 @@ __global__ void __launch_bounds__(kBlock) soa_log_kernel(AdjWork g) {
         b0 = nsplit + __builtin_amdgcn_readfirstlane(b0);
         e0 = min(b0 + qschunk, nq);
       }
-      if (MAM4X_SOA_PRIO && b0 < nlong) __builtin_amdgcn_s_setprio(2);
+      if (b0 < nlong) __builtin_amdgcn_s_setprio(2);
       if (b0 >= nq) {
         exhausted = true;
       } else {

@@ -21,8 +21,10 @@ constexpr int kNBucket = 24;  // half-octave cost buckets: 2 log2(1 + predicted 
 #define MAM4X_QUEUE_CHUNK 64
 #endif
 constexpr int kChunk = MAM4X_QUEUE_CHUNK;  // default queue entries a wave takes per refill
-// First bucket whose waves raise their issue priority (predicted >= ~180
-// sub-steps).
+// Waves whose first chunk comes from buckets >= kLongBucket (predicted >= ~180
+// sub-steps) raise their issue priority: a cell's sub-steps are a serial
+// chain, so the longest cells set the kernel's critical path and should not
+// yield issue slots to the bulk.
 constexpr int kLongBucket = 15;
 // Refills cost a device-scope atomic on a queue counter, and those atomics
 // serialise across the device (tens of ns each), so the kernel keeps their

@@ -41,9 +41,8 @@ def torch_cuda():
 
 
 def run_gpu(torch_cuda, scene, dt=DT, **cfg):
-    """One step on the GPU.  The work-queue schedule is forced (the default
-    picks the fused kernel below 16,384 cells); test_schedules_agree covers
-    the fused kernel."""
+    """One step on the GPU.  The work-queue schedule is forced;
+    test_schedules_agree covers the fused kernel."""
     from mam4xx_amd import _abi
     from mam4xx_amd.chain import Chain, scene_to_device
     torch = torch_cuda
